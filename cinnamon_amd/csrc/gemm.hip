@@ -14,16 +14,20 @@
 // w_fp8.t().contiguous() copy disappears; dgrad/wgrad pass the transposed codes
 // produced by the quantizers.
 //
-// Workgroup tile 128 x 128 x 128, 4 waves in 2 x 2, wave tile 64 x 64.  K blocks
-// are staged global -> registers -> LDS (XOR-swizzled 16-byte chunks, double
-// buffered, one barrier per K block).  The MFMA is issued as B x A^T so each
-// lane ends up holding 4 consecutive columns of one row (one 8-byte bf16 or
-// 16-byte fp32 store per fragment) and a single combined scale sa[m] * sb.
+// The MFMA is issued as B x A^T so each lane ends up holding 4 consecutive columns of
+// one row and a single combined scale sa[m] * sb.  Three families of kernels:
+//   namespaces big and pers  256 x 256 tiles, K % 128 == 0, one tile or several per CU
+//   k_gemm_fp8_bs_tile       any shape: smaller tiles whose K blocks are shared by groups of
+//                            waves (cin_gemm_tile.h)
+//   k_gemm_fp8_bs            128 x 128 tiles with 64-bit addresses, for operands whose rows
+//                            are too far apart for the others' 32-bit offsets: K blocks
+//                            staged global -> registers -> LDS, 4 waves in 2 x 2
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
 
 #include "cin_common.h"
+#include "cin_gemm_tile.h"
 #include "cin_grouped.h"
 #include "cin_runtime.h"
 
@@ -31,8 +35,6 @@ using namespace cin;
 
 namespace {
 
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4v __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 128, BN = 128, BK = 128;
@@ -290,23 +292,6 @@ __device__ inline int sa_row(int q) {
   return (q & ~127) + (((q >> 6) & 1) * 4 + (q & 3)) * 16 + ((q >> 2) & 15);
 }
 
-// 16-byte chunk c of tile row r lives at slot c ^ f(r), f(r) = (r % 8) ^ ((r / 8) % 2):
-// the 8 rows a 32-bank LDS serves together, and the 8 same-parity rows a 64-bank LDS
-// serves together, all hit distinct banks.
-__device__ inline int swz_f(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// DMA of 16 (4) bytes per lane from the buffer to LDS: lane t's bytes land at LDS byte
-// address lds + 16 t (4 t).  lds is wave-uniform.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-}
-// s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima)
-__device__ __forceinline__ void wait_dma() { __builtin_amdgcn_s_waitcnt(0x0F70); }
 // Vector memory operations a wave issues for one K block's DMA: 4 row groups x (A, B), plus
 // the A scales on waves 0-3.  s_waitcnt vmcnt(8): everything but the last 8 has completed.
 constexpr int kDmaOpsPerBlock = 8;
@@ -407,16 +392,6 @@ __device__ __forceinline__ void store_tile(const Tile& T, const v4f (&acc)[8][4]
       }
     }
   }
-}
-
-// s_waitcnt lgkmcnt(0) (vmcnt and expcnt left at their maxima), then a workgroup barrier
-// that the compiler may not move LDS accesses across.  No vmcnt wait: operand DMA stays in
-// flight across it.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
 }
 
 // Read half H of block kb: its four A fragments, and for H = 0 the B fragments and the
@@ -874,21 +849,16 @@ __global__ __launch_bounds__(kThreads, 2) void k_grouped_wgrad_fp8_256(
 // ---------------------------------------------------------------------------
 namespace pers {
 
-using big::dma16;
-using big::dma4;
 using big::kCStride;
 using big::kTileBytes;
 using big::sa_row;
 using big::Smem;
 using big::SmemAll;
-using big::swz_f;
 using big::Tile;
 using big::TK;
 using big::TM;
 using big::TN;
-using big::wait_dma;
 using big::wait_dma_but_block;
-using big::lds_barrier;
 constexpr int kThreads = big::kThreads;
 
 // Scales and expert ranges do not change during a kernel: read through the constant address
@@ -1621,6 +1591,181 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_wgrad_fp8_pers(
 
 }  // namespace pers
 
+// Dense products on cin_gemm_tile.h's tiles.
+template <class C, bool TAIL>
+__global__ __launch_bounds__(C::kThreads) void k_gemm_fp8_bs_tile(
+    const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ sa, int64_t ssam,
+    int64_t ssak, const uint8_t* __restrict__ B, int64_t ldb, const float* __restrict__ sb,
+    int64_t ssbn, int64_t ssbk, int64_t M, int64_t N, int K, void* Cp, int c_dtype, int64_t ldc,
+    uint32_t tiles_m, uint32_t tiles_n) {
+  __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
+  uint32_t tm, tn;
+  big::raster<4>(big::xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * C::TM, n0 = (int64_t)tn * C::TN;
+  gt::Tile t;
+  t.A = A + m0 * lda;
+  t.sa = sa + m0 * ssam;
+  t.B = B + n0 * ldb;
+  t.sb = sb + (n0 >> 7) * ssbn;
+  t.C = static_cast<uint8_t*>(Cp) + (m0 * ldc + n0) * (c_dtype == CIN_DT_F32 ? 4 : 2);
+  t.rows_a = (int)(M - m0 < C::TM ? M - m0 : C::TM);
+  t.rows_b = (int)(N - n0 < C::TN ? N - n0 : C::TN);
+  gt::tile<C, TAIL>(t, lda, ssam, ssak, ldb, ssbk, K, c_dtype, ldc, smem);
+}
+
+// The expert that owns row tile `tile` when every expert's rows are cut into tiles of TM
+// (experts in order): false past the last one.  Each wave looks at 64 experts at a time.
+template <int TM>
+__device__ inline bool find_row_tile(const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E,
+                                     int64_t Tn, int64_t tile, int64_t& e, int64_t& row0, int64_t& row_end) {
+  const int lane = threadIdx.x & 63;
+  int64_t seen = 0;
+  for (int64_t base = 0; base < E; base += 64) {
+    int64_t s0 = 0, s1 = 0;
+    if (base + lane < E) clamp_range(starts, ends, base + lane, Tn, s0, s1);
+    const int64_t n = (s1 - s0 + TM - 1) / TM;
+    int64_t incl = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    const uint64_t past = __ballot(tile < seen + incl);
+    if (past) {
+      const int l = (int)__builtin_ctzll(past);
+      e = base + l;
+      row0 = __shfl(s0, l, 64) + (tile - seen - __shfl(incl - n, l, 64)) * TM;
+      row_end = __shfl(s1, l, 64);
+      return true;
+    }
+    seen += __shfl(incl, 63, 64);
+  }
+  return false;
+}
+
+// Grouped products on the same tiles.
+template <class C, bool TAIL>
+__global__ __launch_bounds__(C::kThreads) void k_grouped_gemm_fp8_tile(
+    const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ sa, int64_t ssam,
+    int64_t ssak, const uint8_t* __restrict__ B, int64_t sbe, int64_t ldb,
+    const float* __restrict__ sb, int64_t ssbe, int64_t ssbn, int64_t ssbk,
+    const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t Tn,
+    int64_t N, int K, void* Cp, int c_dtype, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n) {
+  __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
+  uint32_t tm, tn;
+  big::raster<4>(big::xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
+  int64_t e, row0, row_end;
+  if (!find_row_tile<C::TM>(starts, ends, E, Tn, tm, e, row0, row_end)) return;  // the whole workgroup
+  const int64_t n0 = (int64_t)tn * C::TN;
+  gt::Tile t;
+  t.A = A + row0 * lda;
+  t.sa = sa + row0 * ssam;
+  t.B = B + e * sbe + n0 * ldb;
+  t.sb = sb + e * ssbe + (n0 >> 7) * ssbn;
+  t.C = static_cast<uint8_t*>(Cp) + (row0 * ldc + n0) * (c_dtype == CIN_DT_F32 ? 4 : 2);
+  t.rows_a = __builtin_amdgcn_readfirstlane((int)(row_end - row0 < C::TM ? row_end - row0 : C::TM));
+  t.rows_b = (int)(N - n0 < C::TN ? N - n0 : C::TN);
+  gt::tile<C, TAIL>(t, lda, ssam, ssak, ldb, ssbk, K, c_dtype, ldc, smem);
+}
+
+// Grouped weight gradient on the same tiles (operands and result of pers::
+// k_grouped_wgrad_fp8_pers): dW_e[n, k] reduced over expert e's padded token range, zeros for
+// an expert without tokens.  Workgroups are dispatched in the order of their experts' size,
+// largest first (up to 64 experts; in expert order past that), so that the hardware's own
+// scheduling evens out ragged experts.
+template <class C>
+__global__ __launch_bounds__(C::kThreads) void k_grouped_wgrad_fp8_tile(
+    const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ sa, int64_t ssam,
+    int64_t ssak, const uint8_t* __restrict__ B, int64_t ldb, const float* __restrict__ sb, int64_t ssbm,
+    const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int E, int64_t Tn,
+    int64_t tcap, int64_t M, int64_t N, void* Cp, int c_dtype, int64_t ldc, int64_t sce,
+    uint32_t tiles_m, uint32_t tiles_n) {
+  __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
+  const uint32_t per = tiles_m * tiles_n;
+  const int rank = (int)(blockIdx.x / per);
+  const int lane = threadIdx.x & 63;
+  // expert e of this workgroup, its K blocks and its first padded K block
+  int e = rank, nk = 0;
+  int64_t kb0 = 0;
+  for (int base = 0; base < E; base += 64) {
+    int n = 0;
+    if (base + lane < E) {
+      int64_t s0, s1;
+      clamp_range(starts, ends, base + lane, Tn, s0, s1);
+      n = (int)((s1 - s0 + 127) / 128);
+    }
+    int64_t incl = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int64_t o = __shfl_up(incl, d, 64);
+      if (lane >= d) incl += o;
+    }
+    if (E <= 64) {
+      int before = 0;  // experts ahead of this lane's
+      for (int x = 0; x < E; ++x) {
+        const int o = __builtin_amdgcn_readlane(n, x);
+        before += o > n || (o == n && x < lane) ? 1 : 0;
+      }
+      e = (int)__builtin_ctzll(__ballot(lane < E && before == rank));
+    }
+    if (e < base + 64) {
+      nk = __builtin_amdgcn_readlane(n, e - base);
+      kb0 += __shfl(incl, e - base, 64) - nk;
+      break;
+    }
+    kb0 += __shfl(incl, 63, 64);
+  }
+  // ranges inconsistent with the operands' columns: zero, as for an expert without tokens
+  if ((kb0 + nk) * 128 > tcap) nk = 0;
+  if (nk == 0) kb0 = 0;  // (nothing is read, but the descriptors are built)
+  uint32_t tm, tn;
+  big::raster<4>(blockIdx.x - (uint32_t)rank * per, tiles_m, tiles_n, tm, tn);
+  const int64_t m0 = (int64_t)tm * C::TM, n0 = (int64_t)tn * C::TN;
+  gt::Tile t;
+  t.A = A + m0 * lda + kb0 * 128;
+  t.sa = sa + m0 * ssam + kb0 * ssak;
+  t.B = B + n0 * ldb + kb0 * 128;
+  t.sb = sb + kb0 * ssbm + (n0 >> 7);
+  t.C = static_cast<uint8_t*>(Cp) + ((int64_t)e * sce + m0 * ldc + n0) * (c_dtype == CIN_DT_F32 ? 4 : 2);
+  t.rows_a = (int)(M - m0 < C::TM ? M - m0 : C::TM);
+  t.rows_b = (int)(N - n0 < C::TN ? N - n0 : C::TN);
+  gt::tile<C, false>(t, lda, ssam, ssak, ldb, ssbm, nk * 128, c_dtype, ldc, smem);
+}
+
+// Waves (m, n), MFMA tiles per wave (m, n), K groups.
+using T16x32 = gt::Cfg<1, 2, 1, 1, 8>;
+using T32x32 = gt::Cfg<1, 2, 2, 1, 8>;
+using T32x64 = gt::Cfg<2, 2, 1, 2, 4>;
+using T64x32 = gt::Cfg<2, 2, 2, 1, 4>;
+using T64x64 = gt::Cfg<1, 2, 4, 2, 4>;
+using T64x64Two = gt::Cfg<2, 2, 2, 2, 2>;  // two workgroups fit a CU
+using T128 = gt::Cfg<2, 2, 4, 4, 2>;
+using T128Two = gt::Cfg<4, 2, 2, 4, 1>;    // two workgroups fit a CU
+using T32x128 = gt::Cfg<2, 2, 1, 4, 1>;    // three (grouped products with few rows an expert)
+using T64x128 = gt::Cfg<2, 2, 2, 4, 1>;    // three
+
+// launch(tile type) for an M x N output on ncu CUs.
+// The smallest tile whose grid is at most one workgroup per CU: a smaller one adds CUs and
+// their operand bandwidth, and past one per CU tiles queue.  us with 16x32 / 32x32 / 32x64 /
+// 64x64 tiles: M, N, K = 16, 2048, 7168: 7.4 / 8.4 / 11.3 / 14.3; 48, 4096, 4096: - / 6.9 / 8.3 /
+// 10.0; 200, 1536, 1536: - / 8.7 / 5.6 / 6.3; 768, 768, 4096: - / 17 / 16 / 10.6 (the one
+// serial K loop of 128 x 128 tiles that they replace: 57, 37, 18, 42).  Two 64 x 64
+// workgroups share a CU (1000, 1500, 4000: 18.1 us, 128 x 128 tiles 23.5; past that the other
+// way round: 3000, 1500, 2048: 24.3 against 21.6), and from one round of 128 x 128 tiles on,
+// two of those (8192, 1500, 4000: 71 us against 81 with one).
+template <class F>
+void with_tile(int64_t M, int64_t N, int64_t ncu, F launch) {
+  const auto tiles = [&](int64_t a, int64_t b) { return cdiv(M, a) * cdiv(N, b); };
+  if (tiles(16, 32) <= ncu) return launch(T16x32{});
+  if (tiles(32, 32) <= ncu) return launch(T32x32{});
+  if (tiles(32, 64) <= ncu && tiles(32, 64) <= tiles(64, 32)) return launch(T32x64{});
+  if (tiles(64, 32) <= ncu) return launch(T64x32{});
+  if (tiles(64, 64) <= ncu) return launch(T64x64{});
+  if (tiles(64, 64) <= 2 * ncu) return launch(T64x64Two{});
+  if (tiles(128, 128) <= ncu) return launch(T128{});
+  return launch(T128Two{});
+}
+
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Compute units of the current device (the persistent grid runs one workgroup per CU),
@@ -1656,6 +1801,14 @@ bool big_offsets_fit(int64_t lda, int64_t ldb, int64_t klen, int64_t ssam, int64
   const int64_t nkb = klen / 128 > 0 ? klen / 128 : 1;
   return 255 * lda + klen < lim && 255 * ldb + klen < lim && (255 * ssam + (nkb - 1) * ssak + 1) * 4 < lim;
 }
+
+// Whether a grid of 256 x 256 tiles leaves so many CUs idle in its last round that the 128 x
+// 128 and smaller tiles finish first: at most 5/8 of the rounds' CU slots used.  us, 256 x 256 /
+// smaller tiles: 64 of 256 CUs (4096, 1024, 1024) 14.9 / 11.5 and (2048, 2048, 2048) 24.5 / 16.0;
+// 128 (4096, 2048, 4096) 44.5 / 40.9; 264 (8448, 2048, 2048) 55.8 / 50.4; 320 (10000, 2048, 1024)
+// 33.6 / 31.8; and the other way round: 192 (6144, 2048, 4096) 48.8 / 59.4, 384 (12288, 2048,
+// 2048) 55.0 / 61.4.
+bool rounds_sparse(int64_t tiles, int64_t ncu) { return tiles * 8 <= cdiv(tiles, ncu) * ncu * 5; }
 
 }  // namespace
 
@@ -1694,9 +1847,11 @@ int cin_gemm_fp8_bs(const uint8_t* A, int64_t lda, const float* sa, int64_t ssam
     hipLaunchKernelGGL(k_zero_rows16, grid, 256, 0, s, static_cast<uint16_t*>(C), M, N * es / 2, ldc * es / 2);
     return cin_check_launch("gemm_fp8_bs");
   }
-  if (K % big::TK == 0 && M >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak)) {
+  const uint32_t ncu = (uint32_t)device_cus();
+  const bool tile_fits = gt::offsets_fit(128, lda, ldb, K, ssam, ssak);
+  if (K % big::TK == 0 && M >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak) &&
+      !(tile_fits && rounds_sparse(cdiv(M, big::TM) * cdiv(N, big::TN), ncu))) {
     const uint32_t tm = (uint32_t)cdiv(M, big::TM), tn = (uint32_t)cdiv(N, big::TN);
-    const uint32_t ncu = (uint32_t)device_cus();
     if (tm * tn > ncu) {
       // more tiles than CUs: the persistent walk, whose next tile's DMA overlaps this tile's
       // stores (16-bit C: the fixed-count epilogue).  Every output dtype takes it, so the K
@@ -1718,6 +1873,16 @@ int cin_gemm_fp8_bs(const uint8_t* A, int64_t lda, const float* sa, int64_t ssam
     }
     hipLaunchKernelGGL(big::k_gemm_fp8_bs_256, tm * tn, big::kThreads, 0, s, A, lda, sa, ssam,
                        ssak, B, ldb, sb, ssbn, ssbk, M, N, K, C, c_dtype, ldc, tm, tn);
+    return cin_check_launch("gemm_fp8_bs");
+  }
+  if (tile_fits) {
+    with_tile(M, N, ncu, [&](auto cfg) {
+      using C_ = decltype(cfg);
+      const uint32_t tm = (uint32_t)cdiv(M, C_::TM), tn = (uint32_t)cdiv(N, C_::TN);
+      const auto k = K % 128 == 0 ? k_gemm_fp8_bs_tile<C_, false> : k_gemm_fp8_bs_tile<C_, true>;
+      hipLaunchKernelGGL(k, tm * tn, C_::kThreads, 0, s, A, lda, sa, ssam, ssak, B, ldb, sb, ssbn, ssbk, M, N, (int)K,
+                         C, c_dtype, ldc, tm, tn);
+    });
     return cin_check_launch("gemm_fp8_bs");
   }
   const uint32_t ntn = (uint32_t)cdiv(N, BN);
@@ -1743,12 +1908,52 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
                     aligned16(A) && aligned16(B),
                 "grouped_gemm_fp8: A/B rows must be 16-byte aligned and K-contiguous");
   CIN_CHECK_ARG(ldc >= N, "grouped_gemm_fp8: bad C stride");
-  if (K % big::TK == 0 && T >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak)) {
+  const int64_t ncu = device_cus();
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool big_ok = K % big::TK == 0 && T >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak);
+  if (gt::offsets_fit(128, lda, ldb, K, ssam, ssak)) {
+    const auto launch = [&](auto cfg) {
+      using C_ = decltype(cfg);
+      // sum over experts of ceil(rows / TM) is at most this; surplus workgroups leave at once
+      const int64_t tm = cdiv(T, C_::TM) + E - 1, tn = cdiv(N, C_::TN);
+      const auto k = K % 128 == 0 ? k_grouped_gemm_fp8_tile<C_, false> : k_grouped_gemm_fp8_tile<C_, true>;
+      hipLaunchKernelGGL(k, (unsigned)(tm * tn), C_::kThreads, 0, s, A, lda, sa, ssam, ssak, B, sbe, ldb, sb, ssbe, ssbn,
+                         ssbk, starts, ends, E, T, N, (int)K, C, c_dtype, ldc, (uint32_t)tm, (uint32_t)tn);
+    };
+    CIN_CHECK_ARG(big_ok || (cdiv(T, 128) + E) * cdiv(N, 128) < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
+    if (E == 1) {
+      // one expert: as the dense product of the same shape
+      if (!big_ok || rounds_sparse(cdiv(T, big::TM) * cdiv(N, big::TN), ncu)) {
+        with_tile(T, N, ncu, launch);
+        return cin_check_launch("grouped_gemm_fp8");
+      }
+    } else {
+      // Few rows an expert: the product streams every expert's codes for a fraction of a 256-
+      // row tile, so short tiles, three workgroups a CU.  us, 32 x 128 / 64 x 128 / 128 x 128 / 256 x
+      // 256 tiles at T, E, N, K: 512, 32, 4096, 7168: 224 / 239 / 254 / 274; 1024: 262 / 249 / 281 /
+      // 275; 2048: 352 / 289 / 275 / 274.  With up to 128 rows an expert the 256 x 256 tiles are
+      // half empty; they still win where they fill the chip (4096, 32, 4096, 7168: 418 against
+      // 347), not where about T / 256 + E / 2 row tiles do not (2048, 16, 2048, 1024: 19.8 against
+      // 27.5; 8192, 64, 1024, 512: 28.9 against 35.8).
+      const int64_t rows = T / E;
+      const bool few = (rows < 64 || (rows <= 128 && (T / big::TM + E / 2) * cdiv(N, big::TN) <= ncu)) &&
+                       (cdiv(T, 32) + E) * cdiv(N, 128) < ((int64_t)1 << 31);
+      if (few || !big_ok) {
+        if (!few)
+          launch(T128Two{});
+        else if (rows <= 24)
+          launch(T32x128{});
+        else
+          launch(T64x128{});
+        return cin_check_launch("grouped_gemm_fp8");
+      }
+    }
+  }
+  if (big_ok) {
     const int64_t mt = cdiv(T, big::TM) + E;
     const uint32_t tn = (uint32_t)cdiv(N, big::TN);
     CIN_CHECK_ARG(mt * tn < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
     if (E <= pers::kMaxExpertsLds) {
-      const int64_t ncu = device_cus();
       const unsigned grid = (unsigned)(mt * tn < ncu ? mt * tn : ncu);
 #define CIN_LAUNCH_GROUPED_PERS(EPI_)                                                                \
   hipLaunchKernelGGL(pers::k_grouped_gemm_fp8_pers<EPI_>, grid, big::kThreads, 0,                      \
@@ -1775,7 +1980,6 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
   const int64_t max_tiles = cdiv(T, BM) + E;
   const uint32_t ntn = (uint32_t)cdiv(N, BN);
   CIN_CHECK_ARG(max_tiles * ntn < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
-  hipStream_t s = static_cast<hipStream_t>(stream);
   const unsigned grid = (unsigned)(max_tiles * ntn);
   hipLaunchKernelGGL(k_grouped_gemm_fp8, grid, kThreads, 0, s, A, lda, sa, ssam, ssak, B, sbe, ldb,
                      sb, ssbe, ssbn, ssbk, starts, ends, E, T, N, K, C, c_dtype, ldc, ntn);
@@ -1807,6 +2011,18 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
                 "grouped_wgrad_fp8: operand rows too long for the 256 x 256 tile's 32-bit offsets");
   const int64_t tm = cdiv(N, big::TM), tn = cdiv(K, big::TN);
   CIN_CHECK_ARG(E * tm * tn < ((int64_t)1 << 31), "grouped_wgrad_fp8: grid too large");
+  const int64_t cus = device_cus();
+  if (E == 1 && rounds_sparse(tm * tn, cus) && gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak)) {
+    // one expert: as the dense product of the same shape
+    with_tile(N, K, cus, [&](auto cfg) {
+      using C_ = decltype(cfg);
+      const uint32_t tm_ = (uint32_t)cdiv(N, C_::TM), tn_ = (uint32_t)cdiv(K, C_::TN);
+      hipLaunchKernelGGL(k_grouped_wgrad_fp8_tile<C_>, (unsigned)E * tm_ * tn_, C_::kThreads, 0,
+                         static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, ldb, sb, ssbm, starts, ends,
+                         (int)E, T, tcap, N, K, C, c_dtype, ldc, sce, tm_, tn_);
+    });
+    return cin_check_launch("grouped_wgrad_fp8");
+  }
   const uint32_t ntot = (uint32_t)(E * tm * tn);
   if (E <= pers::kMaxWgradExperts) {
     // one workgroup per CU on the persistent walk; the counted epilogues need every expert's

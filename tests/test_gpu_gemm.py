@@ -70,6 +70,38 @@ def test_gemm_parity(kern, dev, M, N, K):
     assert torch.equal(y16.cpu(), y32.cpu().to(torch.bfloat16)), "bf16 output is not RNE(fp32 output)"
 
 
+# One shape or more for every tile of cin_gemm_tile.h: partial rows, columns and K blocks, K
+# blocks fewer than the groups that share them, and more than 64 per group (the B scales are
+# loaded 64 at a time)
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 16), (15, 4097, 144), (16, 31, 2064), (3, 33, 66048),   # 16 x 32
+    (33, 1000, 1040), (512, 512, 128), (31, 45, 33792),            # 32 x 32 and below
+    (40, 7000, 400), (545, 1000, 272),                             # 32 x 64
+    (1000, 520, 272), (7000, 40, 400),                             # 64 x 32
+    (1000, 1000, 1168), (769, 1025, 528),                          # 64 x 64
+    (1025, 1600, 1168), (2048, 1024, 512),                         # 64 x 64, two per CU
+    (2047, 2040, 656), (4096, 1024, 1024),                         # 128 x 128
+    (2200, 2100, 272), (2049, 8191, 144), (4224, 2176, 384),       # 128 x 128, two per CU
+])
+def test_gemm_tile_edges(kern, dev, M, N, K):
+    xq, xs, wq, ws = _operands(M, N, K, seed=M + N + K)
+    y32, y16 = _run_fp32_and_bf16(kern, dev, xq, xs, wq, ws)
+    want = orc.gemm_ref(xq, xs, wq.view(torch.uint8).t().contiguous(), ws.t().contiguous())
+    _check(y32, want, f"gemm {M}x{N}x{K}")
+    assert torch.equal(y16.cpu(), y32.cpu().to(torch.bfloat16)), "bf16 output is not RNE(fp32 output)"
+
+
+def test_gemm_rows_past_32_bit_offsets(kern, dev):
+    """Rows 2^24 bytes apart: 128 of them pass the 31-bit lane offsets of the tile kernels."""
+    M, N, K = 17, 96, 272
+    xq, xs, wq, ws = _operands(M, N, K, seed=5)
+    far = torch.empty(M, 1 << 24, dtype=torch.uint8, device=dev)[:, :K]
+    far.copy_(xq.view(torch.uint8))
+    y = kern.fp8_gemm_bs(far.view(torch.float8_e4m3fn), xs.to(dev), wq.to(dev), ws.to(dev), torch.float32)
+    want = orc.gemm_ref(xq, xs, wq.view(torch.uint8).t().contiguous(), ws.t().contiguous())
+    _check(y, want, "gemm with distant rows")
+
+
 def test_gemm_against_golden(kern, dev):
     d = np.load(GOLDEN)
     a = torch.from_numpy(d["xc_row_q"]).to(dev)
@@ -255,6 +287,26 @@ def test_grouped_gemm_leaves_rows_outside_ranges(kern, dev, out_dtype):
     assert bool(torch.isnan(got[~covered].float()).all())
     assert torch.equal(got[covered], ref32.cpu()[covered].to(out_dtype))
     _check(ref32.cpu()[covered], want[covered], "grouped with gaps")
+
+
+# The small grouped tiles: rows an expert under and over each tile's height, experts without
+# rows, more than 64 experts (a wave looks them up 64 at a time), partial K blocks and columns
+@pytest.mark.parametrize("counts,N,K", [
+    ([3, 0, 33, 1, 64, 20, 0, 31], 256, 384),            # 32 rows
+    ([0] * 70 + [5, 40, 0, 129] + [2] * 60, 200, 272),
+    ([65, 31, 0, 63, 1, 97], 384, 1024),                 # 64 rows
+    ([200, 0, 129, 90, 1], 100, 400),
+    ([300, 700, 0, 128], 328, 144),                      # 128 rows
+])
+def test_grouped_tile_edges(kern, dev, counts, N, K):
+    from cinnamon_amd import layers
+    xq, xs, wq, ws, starts, ends = _grouped_case(counts, -(-N // 128) * 128, K, seed=len(counts) + K)
+    wq = wq[:, :N]
+    args = [t.to(dev) for t in (xq, xs, wq, ws, starts, ends)]
+    y32 = layers.fp8_grouped_gemm(*args, out_dtype=torch.float32)
+    y16 = layers.fp8_grouped_gemm(*args, out_dtype=torch.bfloat16)
+    _check(y32, orc.grouped_gemm_ref(xq, xs, wq, ws, starts, ends), f"grouped {counts[:8]} {N}x{K}")
+    assert torch.equal(y16.cpu(), y32.cpu().to(torch.bfloat16)), "bf16 output is not RNE(fp32 output)"
 
 
 def test_grouped_equals_dense_for_one_expert(kern, dev):
