@@ -2012,15 +2012,24 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
   const int64_t tm = cdiv(N, big::TM), tn = cdiv(K, big::TN);
   CIN_CHECK_ARG(E * tm * tn < ((int64_t)1 << 31), "grouped_wgrad_fp8: grid too large");
   const int64_t cus = device_cus();
-  if (E == 1 && rounds_sparse(tm * tn, cus) && gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak)) {
-    // one expert: as the dense product of the same shape
-    with_tile(N, K, cus, [&](auto cfg) {
+  // Up to four rounds of 256 x 256 tiles: ragged experts leave the persistent walk waiting for
+  // the CUs that hold the longest tiles (and half-filled rounds), where the 128 x 128 tiles'
+  // dispatch evens them out.  us, persistent / 128 x 128, Zipf(1.1) rows, T, E, N, K: 32768, 16,
+  // 1024, 1024 (1 round) 109 / 61; 32768, 16, 2048, 1024 (2) 135 / 95; 32768, 16, 2048, 2048 (4) 251 /
+  // 232; 65536, 32, 2048, 2048 (8) 426 / 456.
+  if ((E == 1 ? rounds_sparse(tm * tn, cus) : E * tm * tn <= 4 * cus) &&
+      gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak)) {
+    const auto launch = [&](auto cfg) {
       using C_ = decltype(cfg);
       const uint32_t tm_ = (uint32_t)cdiv(N, C_::TM), tn_ = (uint32_t)cdiv(K, C_::TN);
       hipLaunchKernelGGL(k_grouped_wgrad_fp8_tile<C_>, (unsigned)E * tm_ * tn_, C_::kThreads, 0,
                          static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, ldb, sb, ssbm, starts, ends,
                          (int)E, T, tcap, N, K, C, c_dtype, ldc, sce, tm_, tn_);
-    });
+    };
+    if (E == 1)
+      with_tile(N, K, cus, launch);  // as the dense product of the same shape
+    else
+      launch(T128Two{});
     return cin_check_launch("grouped_wgrad_fp8");
   }
   const uint32_t ntot = (uint32_t)(E * tm * tn);

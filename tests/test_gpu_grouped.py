@@ -447,3 +447,61 @@ def test_grouped_wgrad_direct_epilogue(kern, dev, out_dtype):
     for e in range(E):
         assert torch.equal(buf[e * sce:e * sce + N * K].view(N, K), want[e]), f"expert {e}"
         assert float(buf[e * sce + N * K]) == 5.0, f"the element after expert {e}'s block was written"
+
+
+# The 128 x 128 wgrad tiles: partial tiles, experts in size order (up to 64) and in expert order
+@pytest.mark.parametrize("E,T,N,K", [(64, 5000, 304, 256), (70, 5000, 304, 384), (3, 700, 256, 640)])
+def test_grouped_wgrad_tiles(kern, dev, E, T, N, K):
+    from cinnamon_amd import layers
+    counts = _many_expert_counts(E, T, seed=E)
+    starts, ends = _ranges(counts)
+    g = torch.Generator().manual_seed(E)
+    dc = (torch.randn(T, N, generator=g) * 1e-3).to(torch.bfloat16)
+    xq, xs = orc.quant_rowwise(torch.randn(T, K, generator=g).to(torch.bfloat16))
+    dual = orc.grouped_dual_ref(dc, starts, ends)
+    want = orc.grouped_wgrad_ref(dual, orc.grouped_requant_ref(xq, xs, starts, ends), E, N, K)
+    sd, ed = starts.to(dev), ends.to(dev)
+    _, _, qt, st = layers.quantize_fp8_dual_grouped(dc.to(dev), sd, ed)
+    xbt, xblk = layers.requantize_grouped_t(xq.to(dev), xs.to(dev), sd, ed)
+    dw = layers.fp8_grouped_wgrad(qt, st, xbt, xblk, sd, ed, T, out_dtype=torch.float32)
+    _check(dw, want, f"wgrad E={E}")
+    dw16 = layers.fp8_grouped_wgrad(qt, st, xbt, xblk, sd, ed, T, out_dtype=torch.bfloat16)
+    assert torch.equal(dw16, dw.to(torch.bfloat16)), "bf16 wgrad is not RNE(fp32 wgrad)"
+    for e, c in enumerate(counts):
+        if c == 0:
+            assert torch.count_nonzero(dw[e]) == 0, f"expert {e}"
+
+
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_grouped_wgrad_persistent_direct_epilogue(kern, dev, out_dtype):
+    """The same with more than four rounds of 256 x 256 tiles, which the persistent walk takes."""
+    from cinnamon_amd import _lib, layers
+    E, T, N, K = 8, 1500, 3072, 2944
+    starts, ends = _ranges([700, 0, 128, 1, 300, 64, 7, 300])
+    g = torch.Generator().manual_seed(18)
+    dc = (torch.randn(T, N, generator=g) * 1e-3).to(torch.bfloat16).to(dev)
+    xq, xs = kern.quantize_fp8_rowwise(torch.randn(T, K, generator=g).to(torch.bfloat16).to(dev))
+    sd, ed = starts.to(dev), ends.to(dev)
+    _, _, qt, st = layers.quantize_fp8_dual_grouped(dc, sd, ed)
+    xbt, xblk = layers.requantize_grouped_t(xq, xs, sd, ed)
+    want = layers.fp8_grouped_wgrad(qt, st, xbt, xblk, sd, ed, T, out_dtype=out_dtype)
+    sce = N * K + 1
+    buf = torch.full((E * sce,), 5.0, dtype=out_dtype, device=dev)
+    a, b = qt.view(torch.uint8), xbt.view(torch.uint8)
+    _lib.call("cin_grouped_gemm_fp8_wgrad", _lib.ptr(a), a.stride(0), _lib.ptr(st), st.stride(0), st.stride(1),
+              _lib.ptr(b),
+              b.stride(0), _lib.ptr(xblk), xblk.stride(0), _lib.ptr(sd), _lib.ptr(ed), E, T, a.shape[1], N, K,
+              _lib.ptr(buf), _lib.dtype_code(buf), K, sce, _lib.stream_of(a))
+    torch.cuda.synchronize()
+    for e in range(E):
+        assert torch.equal(buf[e * sce:e * sce + N * K].view(N, K), want[e]), f"expert {e}"
+        assert float(buf[e * sce + N * K]) == 5.0, f"the element after expert {e}'s block was written"
+    # expert 0's block (700 tokens, 768 padded) against the dense product of its operands
+    dense = kern.fp8_gemm_bs(qt[:, :768], st[:, :6], xbt[:, :768], xblk[:6].t(), torch.float32)
+    _check(want[0], dense.to(out_dtype).cpu(), "expert 0")
+
+
+@pytest.mark.parametrize("E,T", [(256, 40000), (600, 80000), (4096, 263000), (4100, 263000)])
+def test_grouped_forward_many_experts_long(kern, dev, E, T):
+    """The same with enough rows an expert for the 256-row tiles."""
+    test_grouped_forward_many_experts(kern, dev, E, T)
