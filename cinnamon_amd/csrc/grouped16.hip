@@ -190,31 +190,249 @@ __global__ __launch_bounds__(kThreads) void k_grouped_gemm_f16(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The same product for operands whose rows are 16-byte aligned (K % 8 == 0): workgroup tiles
+// of 16 MT WM x 16 NT WN, K steps of 64 through two LDS stages.  Each thread keeps the next
+// step's operands in flight in registers, in their own dtype, while the current step's MFMAs
+// run, then converts them to fp16 on the way into LDS: no converted copy of the weights is
+// ever stored.  A wider tile reads fp32 weights less often: with 256 x 256 tiles a step's 96 KB
+// of operands (fp32 weights, 16-bit rows) take about 1500 cycles at 64 B / clk and its MFMAs
+// 2048, with 128 x 128 tiles 768 and 512.  Rows past an expert or past N and elements past K
+// come from out-of-range lanes, which read as zero.  32768 Zipf rows, 16 experts, 2048 x 1024,
+// bf16 rows: 217 us with fp32 weights, 174 with bf16 (k_grouped_gemm_f16 400 and 280, the same
+// bits): 0.63 and 0.79 PFLOP/s, with 1088 tiles in five rounds of 256.
+// ---------------------------------------------------------------------------
+typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+constexpr uint32_t kOut = 0x80000000u;  // an out-of-range lane offset
+
+__device__ inline h2 to_h2(float a, float b) { return __builtin_convertvector(f2{a, b}, h2); }
+
+// One operand's share of a K step: ROWS rows x 64 elements over THREADS threads, 16 bytes of
+// the source dtype per thread and operation.
+template <int DT, int ROWS, int THREADS>
+struct Operand {
+  static constexpr int kEs = DT == CIN_DT_F32 ? 4 : 2;
+  static constexpr int kLanes = 64 * kEs / 16;  // threads of one row
+  static constexpr int kOps = ROWS * kLanes / THREADS;
+  static constexpr int kRowsPerOp = THREADS / kLanes;
+  static_assert(ROWS * kLanes % THREADS == 0 && kRowsPerOp % 16 == 0, "whole operations, one swizzle per thread");
+  v4u r[kOps];
+  __amdgpu_buffer_rsrc_t rsrc;
+  uint32_t off, step;
+  uint32_t lds;  // byte offset of operation 0 in a stage
+  int k;         // first element of the thread's 16 bytes within a step
+
+  __device__ __forceinline__ void init(const void* p, int64_t ld, int rows, int64_t K, int tid) {
+    rsrc = make_rsrc(p, ((int64_t)(rows - 1) * ld + K) * kEs);
+    const int row = tid / kLanes, c = tid % kLanes;
+    k = c * (16 / kEs);
+    off = (uint32_t)(row * ld * kEs) + c * 16;
+    step = (uint32_t)(kRowsPerOp * ld * kEs);
+    const int chunk = DT == CIN_DT_F32 ? c >> 1 : c;
+    lds = (uint32_t)(row * kRowBytes + ((chunk ^ swz_f(row)) << 4) + (DT == CIN_DT_F32 ? (c & 1) * 8 : 0));
+  }
+  __device__ __forceinline__ void fetch(int64_t k0, int64_t K) {
+    const uint32_t out = k0 + k < K ? 0u : kOut;
+#pragma unroll
+    for (int i = 0; i < kOps; ++i)
+      r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (off + i * step) | out, (uint32_t)(k0 * kEs), 0);
+  }
+  __device__ __forceinline__ void store(uint8_t* stage) const {
+#pragma unroll
+    for (int i = 0; i < kOps; ++i) {
+      uint8_t* d = stage + lds + i * kRowsPerOp * kRowBytes;
+      if constexpr (DT == CIN_DT_F32) {
+        const h2 a = to_h2(__uint_as_float(r[i][0]), __uint_as_float(r[i][1]));
+        const h2 b = to_h2(__uint_as_float(r[i][2]), __uint_as_float(r[i][3]));
+        *reinterpret_cast<h4*>(d) = h4{a[0], a[1], b[0], b[1]};
+      } else if constexpr (DT == CIN_DT_F16) {
+        *reinterpret_cast<v4u*>(d) = r[i];
+      } else {
+        h8 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const h2 a = to_h2(bf16_lo(r[i][e]), bf16_hi(r[i][e]));
+          o[2 * e] = a[0];
+          o[2 * e + 1] = a[1];
+        }
+        *reinterpret_cast<h8*>(d) = o;
+      }
+    }
+  }
+};
+
+template <int WM_, int WN_, int MT_, int NT_>
+struct Cfg16 {
+  static constexpr int WM = WM_, WN = WN_, MT = MT_, NT = NT_;
+  static constexpr int kThreads = 64 * WM * WN, TM = 16 * MT * WM, TN = 16 * NT * WN;
+  static constexpr int kStage = (TM + TN) * kRowBytes;
+  static constexpr int kCStride = TN * 2 + 16;  // bytes; rows 4 banks apart
+  static constexpr int kBytes = 2 * kStage > TM * kCStride ? 2 * kStage : TM * kCStride;
+};
+using W256 = Cfg16<2, 4, 8, 4>;    // 8 waves of 128 x 64
+using W128 = Cfg16<4, 2, 2, 4>;    // 8 waves of 32 x 64, two workgroups a CU
+using W64x128 = Cfg16<2, 2, 2, 4>; // 4 waves of 32 x 64, three workgroups a CU
+
+template <class C, int ADT, int BDT>
+__global__ __launch_bounds__(C::kThreads, 2) void k_grouped_gemm_f16_tile(
+    const void* __restrict__ A, int64_t lda, const void* __restrict__ B, int64_t sbe, int64_t ldb,
+    const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t T,
+    int64_t N, int64_t K, _Float16* __restrict__ Cp, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n) {
+  __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
+  constexpr int MT = C::MT, NT = C::NT;
+  // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of tiles, four row tiles
+  // (mostly one expert's) against one column tile after another
+  const uint32_t G = gridDim.x, Gf = G & ~7u, b0 = blockIdx.x;
+  const uint32_t b = b0 < Gf ? (b0 & 7u) * (Gf >> 3) + (b0 >> 3) : b0;
+  const uint32_t grp = b / (4 * tiles_n), first = grp * 4;
+  const uint32_t gm = tiles_m - first < 4 ? tiles_m - first : 4, w = b - grp * 4 * tiles_n;
+  const uint32_t tm = first + w % gm, tn = w / gm;
+  int64_t e, r0, r1;
+  if (!find_row_tile<C::TM>(starts, ends, E, T, tm, e, r0, r1)) return;  // the whole workgroup
+  const int nr = __builtin_amdgcn_readfirstlane((int)(r1 - r0 < C::TM ? r1 - r0 : C::TM));
+  const int64_t n0 = (int64_t)tn * C::TN;
+  const int nc = (int)(N - n0 < C::TN ? N - n0 : C::TN);
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / C::WN, wn = wave % C::WN;
+  const int l16 = lane & 15, kq = lane >> 4;
+  Operand<ADT, C::TM, C::kThreads> oa;
+  Operand<BDT, C::TN, C::kThreads> ob;
+  oa.init(static_cast<const uint8_t*>(A) + r0 * lda * oa.kEs, lda, nr, K, tid);
+  ob.init(static_cast<const uint8_t*>(B) + (e * sbe + n0 * ldb) * ob.kEs, ldb, nc, K, tid);
+  const int fsw = swz_f(l16);
+  const uint32_t fa = (uint32_t)((wm * 16 * MT + l16) * kRowBytes);
+  const uint32_t fb = (uint32_t)((C::TM + wn * 16 * NT + l16) * kRowBytes);
+
+  v4f acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  const int nkt = (int)((K + BK - 1) / BK);
+  // half of a K step: 32 elements
+  auto half = [&](const uint8_t* st, int ks) {
+    const uint32_t ck = (uint32_t)(((4 * ks + kq) ^ fsw) << 4);
+    h8 bfr[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) bfr[j] = *reinterpret_cast<const h8*>(st + fb + j * 16 * kRowBytes + ck);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const h8 afr = *reinterpret_cast<const h8*>(st + fa + i * 16 * kRowBytes + ck);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bfr[j], afr, acc[i][j], 0, 0, 0);
+    }
+  };
+  oa.fetch(0, K);
+  ob.fetch(0, K);
+  oa.store(smem);
+  ob.store(smem + C::TM * kRowBytes);
+  if (nkt > 1) {
+    oa.fetch(BK, K);
+    ob.fetch(BK, K);
+  }
+  __syncthreads();
+  for (int kt = 0; kt < nkt; ++kt) {
+    const uint8_t* st = smem + (kt & 1) * C::kStage;
+    half(st, 0);
+    if (kt + 1 < nkt) {
+      // step kt + 1, in flight since step kt - 1, into the stage read last in that step
+      uint8_t* nx = smem + ((kt + 1) & 1) * C::kStage;
+      oa.store(nx);
+      ob.store(nx + C::TM * kRowBytes);
+      if (kt + 2 < nkt) {
+        oa.fetch((int64_t)(kt + 2) * BK, K);
+        ob.fetch((int64_t)(kt + 2) * BK, K);
+      }
+    }
+    half(st, 1);
+    __syncthreads();
+  }
+  // fp16 rows through LDS: a lane holds C[m = l16][n = 4 kq .. + 3]
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const h2 a = to_h2(acc[i][j][0], acc[i][j][1]), c = to_h2(acc[i][j][2], acc[i][j][3]);
+      *reinterpret_cast<h4*>(smem + (wm * 16 * MT + i * 16 + l16) * C::kCStride + (wn * 16 * NT + j * 16 + kq * 4) * 2) =
+          h4{a[0], a[1], c[0], c[1]};
+    }
+  __syncthreads();
+  constexpr int kChunks = C::TN / 8;
+  for (int q = tid; q < C::TM * kChunks; q += C::kThreads) {
+    const int m = q / kChunks, n = (q % kChunks) * 8;
+    if (m >= nr || n >= nc) continue;
+    _Float16* cp = Cp + (r0 + m) * ldc + n0 + n;
+    const h8 v = *reinterpret_cast<const h8*>(smem + m * C::kCStride + n * 2);
+    if (n + 8 <= nc && (((uintptr_t)cp) & 15) == 0)
+      *reinterpret_cast<h8*>(cp) = v;
+    else
+      for (int r = 0; r < 8; ++r)
+        if (n + r < nc) cp[r] = v[r];
+  }
+}
+
 inline bool valid_dtype(int dt) { return dt == CIN_DT_BF16 || dt == CIN_DT_F32 || dt == CIN_DT_F16; }
 inline int elem_size(int dt) { return dt == CIN_DT_F32 ? 4 : 2; }
 
+struct Args {
+  const void* A;
+  int64_t lda;
+  const void* B;
+  int64_t sbe, ldb;
+  const int64_t *starts, *ends;
+  int64_t E, T, N, K;
+  _Float16* C;
+  int64_t ldc;
+};
+
+template <class C, int ADT, int BDT>
+void launch_tile(const Args& a, hipStream_t s) {
+  const int64_t tm = cdiv(a.T, C::TM) + a.E - 1, tn = cdiv(a.N, C::TN);
+  hipLaunchKernelGGL((k_grouped_gemm_f16_tile<C, ADT, BDT>), (unsigned)(tm * tn), C::kThreads, 0, s, a.A, a.lda, a.B,
+                     a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C, a.ldc, (uint32_t)tm, (uint32_t)tn);
+}
+
 template <int ADT, int BDT>
-void launch(bool vec, unsigned grid, hipStream_t s, const void* A, int64_t lda, const void* B,
-            int64_t sbe, int64_t ldb, const int64_t* starts, const int64_t* ends, int64_t E,
-            int64_t T, int64_t N, int64_t K, _Float16* C, int64_t ldc, uint32_t tiles_n) {
-  if (vec)
-    hipLaunchKernelGGL((k_grouped_gemm_f16<ADT, BDT, true>), grid, kThreads, 0, s, A, lda, B, sbe,
-                       ldb, starts, ends, E, T, N, K, C, ldc, tiles_n);
-  else
-    hipLaunchKernelGGL((k_grouped_gemm_f16<ADT, BDT, false>), grid, kThreads, 0, s, A, lda, B, sbe,
-                       ldb, starts, ends, E, T, N, K, C, ldc, tiles_n);
+void launch(const Args& a, hipStream_t s) {
+  const int ea = elem_size(ADT), eb = elem_size(BDT);
+  const bool rows16 = ((uintptr_t)a.A % 16) == 0 && ((uintptr_t)a.B % 16) == 0 && (a.lda * ea) % 16 == 0 &&
+                      (a.ldb * eb) % 16 == 0 && (a.sbe * eb) % 16 == 0;
+  const int64_t lim = (int64_t)1 << 31;  // lane offsets from a tile's first row
+  if (rows16 && a.K > 0 && a.K % 8 == 0 && (256 * a.lda + a.K) * ea < lim && (256 * a.ldb + a.K) * eb < lim) {
+    // us, 256 x 256 / 128 x 128 / 64 x 128 tiles, fp32 and bf16 weights, T, E, N, K: 32768, 16, 2048,
+    // 1024 (four rounds of 256 x 256): 217, 174 / 236, 208 / 297, 240; 16384 (two): 120, 109 / 120,
+    // 105 / 151, 123; 8192 (one): 76, 67 / 69, 60 / 86, 69; 1024 (64 rows an expert): 37, 34 / 31, 24 /
+    // 33, 19; 64: 37, 34 / 22, 17 / 22, 15.
+    if (a.T / 256 * cdiv(a.N, 256) >= 512)
+      launch_tile<W256, ADT, BDT>(a, s);
+    else if (a.T <= 64 * a.E && (cdiv(a.T, 64) + a.E) * cdiv(a.N, 128) < lim)
+      launch_tile<W64x128, ADT, BDT>(a, s);
+    else
+      launch_tile<W128, ADT, BDT>(a, s);
+    return;
+  }
+  const int64_t tn = cdiv(a.N, BN);
+  const unsigned grid = (unsigned)((cdiv(a.T, BM) + a.E) * tn);
+  // whole 32-element vector loads where rows and K steps are aligned
+  const auto k = rows16 && a.K % BK == 0 ? k_grouped_gemm_f16<ADT, BDT, true> : k_grouped_gemm_f16<ADT, BDT, false>;
+  hipLaunchKernelGGL(k, grid, kThreads, 0, s, a.A, a.lda, a.B, a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C,
+                     a.ldc, (uint32_t)tn);
 }
 
 template <int ADT>
-void launch_b(int b_dtype, bool vec, unsigned grid, hipStream_t s, const void* A, int64_t lda,
-              const void* B, int64_t sbe, int64_t ldb, const int64_t* starts, const int64_t* ends,
-              int64_t E, int64_t T, int64_t N, int64_t K, _Float16* C, int64_t ldc, uint32_t tn) {
+void launch_b(int b_dtype, const Args& a, hipStream_t s) {
   if (b_dtype == CIN_DT_BF16)
-    launch<ADT, CIN_DT_BF16>(vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, C, ldc, tn);
+    launch<ADT, CIN_DT_BF16>(a, s);
   else if (b_dtype == CIN_DT_F16)
-    launch<ADT, CIN_DT_F16>(vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, C, ldc, tn);
+    launch<ADT, CIN_DT_F16>(a, s);
   else
-    launch<ADT, CIN_DT_F32>(vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, C, ldc, tn);
+    launch<ADT, CIN_DT_F32>(a, s);
 }
 
 }  // namespace
@@ -230,22 +448,15 @@ int cin_grouped_gemm_f16(const void* A, int a_dtype, int64_t lda, const void* B,
   if (E == 0 || T == 0 || N == 0) return CIN_OK;
   CIN_CHECK_ARG(A && B && starts && ends && C, "grouped_gemm_f16: null pointer");
   CIN_CHECK_ARG(lda >= K && ldb >= K && ldc >= N && sbe >= 0, "grouped_gemm_f16: bad strides");
-  // full 32-element vector loads need every row and tile start aligned to the vector
-  const int ea = elem_size(a_dtype), eb = elem_size(b_dtype);
-  const bool vec = K % BK == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)B % 16) == 0 &&
-                   (lda * ea) % 16 == 0 && (ldb * eb) % 16 == 0 && (sbe * eb) % 16 == 0;
-  const int64_t tiles = cdiv(T, BM) + E;
-  const int64_t tn = cdiv(N, BN);
-  CIN_CHECK_ARG(tiles * tn < ((int64_t)1 << 31), "grouped_gemm_f16: grid too large");
-  const unsigned grid = (unsigned)(tiles * tn);
+  CIN_CHECK_ARG((cdiv(T, BM) + E) * cdiv(N, BN) < ((int64_t)1 << 31), "grouped_gemm_f16: grid too large");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  _Float16* Ch = static_cast<_Float16*>(C);
+  const Args a = {A, lda, B, sbe, ldb, starts, ends, E, T, N, K, static_cast<_Float16*>(C), ldc};
   if (a_dtype == CIN_DT_BF16)
-    launch_b<CIN_DT_BF16>(b_dtype, vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, Ch, ldc, (uint32_t)tn);
+    launch_b<CIN_DT_BF16>(b_dtype, a, s);
   else if (a_dtype == CIN_DT_F16)
-    launch_b<CIN_DT_F16>(b_dtype, vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, Ch, ldc, (uint32_t)tn);
+    launch_b<CIN_DT_F16>(b_dtype, a, s);
   else
-    launch_b<CIN_DT_F32>(b_dtype, vec, grid, s, A, lda, B, sbe, ldb, starts, ends, E, T, N, K, Ch, ldc, (uint32_t)tn);
+    launch_b<CIN_DT_F32>(b_dtype, a, s);
   return cin_check_launch("grouped_gemm_f16");
 }
 

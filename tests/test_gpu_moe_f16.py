@@ -51,3 +51,31 @@ def test_grouped_f16_parity(kern, dev, xdt, wdt, N, K):
         inside[s:t] = True
     got, want = out[inside].double(), ref[inside]
     assert (got - want).abs().max() / want.abs().max() <= 1e-3
+
+
+# Every tile of the aligned path (64 x 128, 128 x 128, 256 x 256): partial rows, columns and K
+# steps, one K step, experts without rows, more than 64 experts; and against the general kernel
+# (unaligned rows), whose sums it repeats in the same order
+@pytest.mark.parametrize("counts,N,K", [
+    ([3, 0, 65, 1, 40], 136, 8), ([2] * 66 + [0, 100], 200, 200),
+    ([300, 0, 128, 1, 555, 64, 0, 1000], 328, 520),
+    ([9000, 0, 257, 7127, 1], 2120, 72),
+])
+@pytest.mark.parametrize("xdt,wdt", [(torch.bfloat16, torch.float32), (torch.float16, torch.bfloat16),
+                                     (torch.float32, torch.float16)])
+def test_grouped_f16_tiles(kern, dev, counts, N, K, xdt, wdt):
+    ends = torch.tensor(counts).cumsum(0).to(dev)
+    starts = ends - torch.tensor(counts, device=dev)
+    T, E = sum(counts), len(counts)
+    g = torch.Generator(device=dev).manual_seed(N + K)
+    x = torch.randn(T, K, generator=g, device=dev).to(xdt)
+    w = (torch.randn(E, N, K, generator=g, device=dev) * 0.05).to(wdt)
+    out = kern.moe_grouped_gemm(x, w, starts, ends)
+    wide = torch.zeros(T, K + 1, dtype=xdt, device=dev)
+    wide[:, :K] = x
+    general = kern.moe_grouped_gemm(wide[:, :K], w, starts, ends)
+    assert torch.equal(out, general)
+    # fp32 sums of exact fp16 products (2^-24 a term) and one fp16 rounding (2^-11)
+    want = torch.cat([x[a:b].half().double() @ w[e].half().double().t()
+                      for e, (a, b) in enumerate(zip(starts.tolist(), ends.tolist()))])
+    assert ((out.double() - want).abs() <= 2 ** -10 * want.abs() + K * 2 ** -22 * want.abs().max()).all()
