@@ -540,10 +540,12 @@ struct TileGeo {
   int tw;       // transposed columns written: nr (dense) or 128 (padded axis)
 };
 
-// Dense tiles: t -> (row block t / nbc, column block cb0 + t % nbc).
+// Dense tiles: t -> (row block t / nbc, column block cb0 + t % nbc).  pad: the transposed outputs
+// are written in whole 128-column tiles, zeros past row M.
 struct DenseTiles {
   int64_t M;
   uint32_t nbc, cb0;
+  bool pad = false;
   __device__ void operator()(uint32_t t, TileGeo& g) const {
     const uint32_t rb = t / nbc;
     g.cb = cb0 + (t - rb * nbc);
@@ -551,7 +553,7 @@ struct DenseTiles {
     const int64_t left = M - g.r0;
     g.nr = (int)(left < 128 ? left : 128);
     g.t0 = g.r0;
-    g.tw = g.nr;
+    g.tw = pad ? 128 : g.nr;
   }
 };
 
@@ -563,6 +565,7 @@ struct DenseTiles {
 struct DenseTilesCM {
   int64_t M;
   uint32_t nrb, cb0;
+  bool pad = false;
   __device__ void operator()(uint32_t t, TileGeo& g) const {
     const uint32_t cbl = t / nrb;
     const uint32_t rb = t - cbl * nrb;
@@ -571,7 +574,7 @@ struct DenseTilesCM {
     const int64_t left = M - g.r0;
     g.nr = (int)(left < 128 ? left : 128);
     g.t0 = g.r0;
-    g.tw = g.nr;
+    g.tw = pad ? 128 : g.nr;
   }
 };
 
@@ -1193,9 +1196,9 @@ __global__ __launch_bounds__(kThreads, (DT == CIN_DT_F32 && !EDGE) ? 3 : 1) void
                                                       int64_t ssm, int64_t ssk, uint8_t* qt,
                                                       int64_t sqtm, int vec_t, float* st,
                                                       int64_t sstm, int64_t sstk, uint32_t nbc,
-                                                      uint32_t cb0, uint32_t ntiles) {
+                                                      uint32_t cb0, uint32_t ntiles, int pad) {
   __shared__ DualSmem sm;
-  DenseTiles geo{M, nbc, cb0};
+  DenseTiles geo{M, nbc, cb0, pad != 0};
   dual_run<DT, EDGE>(geo, ntiles, x, N, sxm, round_scale != 0, q, sqm, s, ssm, ssk, qt, sqtm,
                      vec_t != 0, st, sstm, sstk, sm);
 }
@@ -1449,10 +1452,10 @@ __global__ __launch_bounds__(kThreads, 5) void k_requant128(const uint8_t* __res
                                                          int64_t ssm, int64_t ssk, uint8_t* qb, int64_t sqbm,
                                                          uint8_t* qbt, int64_t sqbtm, int vec_t,
                                                          float* sblk, int64_t ssbm, uint32_t nbc,
-                                                         uint32_t cb0, uint32_t ntiles) {
+                                                         uint32_t cb0, uint32_t ntiles, int pad) {
   __shared__ RequantSmem sm;
   (void)nbc;
-  DenseTilesCM geo{M, (uint32_t)((M + 127) >> 7), cb0};
+  DenseTilesCM geo{M, (uint32_t)((M + 127) >> 7), cb0, pad != 0};
   requant_run<EDGE>(geo, ntiles, q, K, sqm, srow, ssm, ssk, qb, sqbm, qbt, sqbtm, vec_t != 0, sblk,
                     ssbm, sm);
 }
@@ -1491,12 +1494,12 @@ __global__ __launch_bounds__(kThreads, 5) void k_quant_bwd(
     int64_t sqm, float* s, int64_t ssm, int64_t ssk, uint8_t* qt, int64_t sqtm, int dvec_t, float* st,
     int64_t sstm, int64_t sstk, const uint8_t* __restrict__ xq, int64_t K, int64_t sxqm,
     const float* __restrict__ srow, int64_t ssrm, int64_t ssrk, uint8_t* xbt, int64_t sxbtm, int rvec_t, float* sblk, int64_t ssbm, uint32_t nd,
-    uint32_t ntiles) {
+    uint32_t ntiles, int pad) {
   static_assert(DT != CIN_DT_F32, "the pair launch takes 16-bit dY");
   __shared__ BwdSmem sm;
   uint32_t t = blockIdx.x;
   {
-    const DenseTiles dgeo{M, (uint32_t)(N >> 7), 0};
+    const DenseTiles dgeo{M, (uint32_t)(N >> 7), 0, pad != 0};
     for (; t < nd; t += gridDim.x) {
       TileGeo g;
       dgeo(t, g);
@@ -1507,7 +1510,7 @@ __global__ __launch_bounds__(kThreads, 5) void k_quant_bwd(
     }
   }
   __syncthreads();  // the union's other member: every thread is past its dual tiles
-  const DenseTilesCM rgeo{M, (uint32_t)((M + 127) >> 7), 0};
+  const DenseTilesCM rgeo{M, (uint32_t)((M + 127) >> 7), 0, pad != 0};
   for (; t < ntiles; t += gridDim.x) {
     TileGeo g;
     rgeo(t - nd, g);
@@ -1784,6 +1787,16 @@ __global__ __launch_bounds__(kThreads) void k_indexer_quant2(const void* __restr
     rowwise128_body<DT, 8, 1, FULL, kMapFirstScale>(blockIdx.x - gk, gridDim.x - gk, q, d, d, 0, q8, d, qs, 1, 0,
                                                     nb, ntq, nullptr, 1, 0);
 }
+
+namespace {
+// qt[r, c0 .. c0 + w) = 0 for r < rows.
+__global__ __launch_bounds__(kThreads) void k_zero_cols(uint8_t* __restrict__ qt, int64_t ld, int64_t rows, int64_t c0,
+                                                        int w) {
+  const int64_t n = rows * w;
+  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads)
+    qt[i / w * ld + c0 + i % w] = 0;
+}
+}  // namespace
 
 extern "C" {
 
@@ -2108,9 +2121,10 @@ int cin_dequant(const uint8_t* q, int64_t M, int64_t N, int64_t sqm, int64_t sqn
   return cin_check_launch("dequant");
 }
 
-int cin_quant_dual(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm, int64_t sdn,
-                   int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
-                   uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk, void* stream) {
+// pad: qt's columns [M, 128 ceil(M / 128)) are written too, as zeros.
+static int quant_dual(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm, int64_t sdn,
+                      int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                      uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk, bool pad, void* stream) {
   CIN_CHECK_ARG(valid_dtype(dy_dtype), "quant_dual: unsupported dtype %d", dy_dtype);
   CIN_CHECK_ARG(M >= 0 && N >= 0, "quant_dual: negative shape");
   if (M == 0 || N == 0) return CIN_OK;
@@ -2133,7 +2147,7 @@ int cin_quant_dual(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t s
     hipLaunchKernelGGL((k_dual128<DT, EDGE>), grid_, kThreads, 0,                              \
                        stream_, dy, M, N, sdm, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, vec_t, \
                        st, sstm, sstk,                                                         \
-                       (uint32_t)(NBC), (uint32_t)(CB0), nt);                                  \
+                       (uint32_t)(NBC), (uint32_t)(CB0), nt, (int)pad);                        \
   } while (0)
 #define CIN_DUAL128_ALL(DT)                                   \
   do {                                                        \
@@ -2153,8 +2167,19 @@ int cin_quant_dual(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t s
   // Strided input: two generic row-wise passes (dy, then dy^T through strides).
   int rc = cin_quant_rowwise(dy, dy_dtype, M, N, sdm, sdn, 128, round_scale, q, sqm, s, ssm, ssk, stream);
   if (rc != CIN_OK) return rc;
-  return cin_quant_rowwise(dy, dy_dtype, N, M, sdn, sdm, 128, round_scale, qt, sqtm, st, sstm, sstk,
-                           stream);
+  rc = cin_quant_rowwise(dy, dy_dtype, N, M, sdn, sdm, 128, round_scale, qt, sqtm, st, sstm, sstk, stream);
+  if (rc != CIN_OK || !pad || M % 128 == 0) return rc;
+  const int64_t n = N * (128 - M % 128);
+  hipLaunchKernelGGL(k_zero_cols, (unsigned)(cdiv(n, kThreads) < 65536 ? cdiv(n, kThreads) : 65536), kThreads, 0,
+                     stream_, qt, sqtm, N, M, 128 - (int)(M % 128));
+  return cin_check_launch("quant_dual");
+}
+
+int cin_quant_dual(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm, int64_t sdn,
+                   int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                   uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk, void* stream) {
+  return quant_dual(dy, dy_dtype, M, N, sdm, sdn, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, st, sstm, sstk, false,
+                    stream);
 }
 
 int cin_quant_dual_grouped(const void* dy, int dy_dtype, int64_t T, int64_t N, int64_t sdm,
@@ -2275,10 +2300,10 @@ int cin_requant_row_to_block_grouped(const uint8_t* q, int64_t T, int64_t K, int
   return cin_check_launch("requant_row_to_block_grouped");
 }
 
-int cin_requant_row_to_block(const uint8_t* q, int64_t M, int64_t K, int64_t sqm,
-                             const float* srow, int64_t ssm, int64_t ssk, uint8_t* qb,
-                             int64_t sqbm, uint8_t* qbt, int64_t sqbtm, float* sblk, int64_t ssbm,
-                             void* stream) {
+// pad: qbt's columns [M, 128 ceil(M / 128)) are written too, as zeros.
+static int requant(const uint8_t* q, int64_t M, int64_t K, int64_t sqm, const float* srow, int64_t ssm, int64_t ssk,
+                   uint8_t* qb, int64_t sqbm, uint8_t* qbt, int64_t sqbtm, float* sblk, int64_t ssbm, bool pad,
+                   void* stream) {
   CIN_CHECK_ARG(M >= 0 && K >= 0, "requant: negative shape");
   if (M == 0 || K == 0) return CIN_OK;
   CIN_CHECK_ARG(q && srow && sblk && (qb || qbt), "requant: null pointer");
@@ -2299,7 +2324,7 @@ int cin_requant_row_to_block(const uint8_t* q, int64_t M, int64_t K, int64_t sqm
     const unsigned grid_ = resident_grid<k_requant128<EDGE>>(nt);                               \
     hipLaunchKernelGGL(k_requant128<EDGE>, grid_, kThreads, 0, s, q,                            \
                        M, K, sqm, srow, ssm, ssk, qb, sqbm, qbt, sqbtm, vec_t, sblk, ssbm, (uint32_t)(NBC), \
-                       (uint32_t)(CB0), nt);                                                    \
+                       (uint32_t)(CB0), nt, (int)pad);                                          \
   } while (0)
   if (nfull > 0) CIN_REQ(false, nfull, 0);
   if (K % 128 != 0) CIN_REQ(true, 1, nfull);
@@ -2307,21 +2332,30 @@ int cin_requant_row_to_block(const uint8_t* q, int64_t M, int64_t K, int64_t sqm
   return cin_check_launch("requant_row_to_block");
 }
 
-int cin_quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm,
-                       int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
-                       uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk,
-                       const uint8_t* xq, int64_t K, int64_t sxqm, const float* xs, int64_t sxsm,
-                       int64_t sxsk, uint8_t* xbt, int64_t sxbtm, float* sblk, int64_t ssbm,
-                       void* stream) {
+int cin_requant_row_to_block(const uint8_t* q, int64_t M, int64_t K, int64_t sqm,
+                             const float* srow, int64_t ssm, int64_t ssk, uint8_t* qb,
+                             int64_t sqbm, uint8_t* qbt, int64_t sqbtm, float* sblk, int64_t ssbm,
+                             void* stream) {
+  return requant(q, M, K, sqm, srow, ssm, ssk, qb, sqbm, qbt, sqbtm, sblk, ssbm, false, stream);
+}
+
+// pad: qt and xbt have their columns [M, 128 ceil(M / 128)) written too, as zeros.
+static int quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm,
+                          int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                          uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk,
+                          const uint8_t* xq, int64_t K, int64_t sxqm, const float* xs, int64_t sxsm,
+                          int64_t sxsk, uint8_t* xbt, int64_t sxbtm, float* sblk, int64_t ssbm, bool pad,
+                          void* stream) {
   CIN_CHECK_ARG(valid_dtype(dy_dtype), "quant_backward: unsupported dtype %d", dy_dtype);
   CIN_CHECK_ARG(M >= 0 && N >= 0 && K >= 0, "quant_backward: negative shape");
   if (M == 0 || (N == 0 && K == 0)) return CIN_OK;
   CIN_CHECK_ARG(dy && q && s && qt && st && xq && xs && xbt && sblk, "quant_backward: null pointer");
-  CIN_CHECK_ARG(sqm >= N && sqtm >= M && scale_layout_ok(M, cdiv(N, 128), ssm, ssk) &&
+  const int64_t cols_t = pad ? 128 * cdiv(M, 128) : M;
+  CIN_CHECK_ARG(sqm >= N && sqtm >= cols_t && scale_layout_ok(M, cdiv(N, 128), ssm, ssk) &&
                     scale_layout_ok(N, cdiv(M, 128), sstm, sstk),
                 "quant_backward: dY output row stride too small or scale strides overlap");
   CIN_CHECK_ARG(aligned(xq, 8) && sxqm % 8 == 0 && sxqm >= K && scale_layout_ok(M, cdiv(K, 128), sxsm, sxsk) &&
-                    sxbtm >= M && ssbm >= cdiv(K, 128),
+                    sxbtm >= cols_t && ssbm >= cdiv(K, 128),
                 "quant_backward: bad X codes, scales or outputs");
   const int es = elem_size(dy_dtype);
   // one launch: 16-bit dY and both widths whole 128-column blocks, with the layouts the two
@@ -2332,11 +2366,10 @@ int cin_quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64
                     tile_fits32(sqm) && tile_fits32(sxqm) && tile_fits32(sxsm * 4) &&
                     cdiv(M, 128) * (N / 128 + K / 128) < ((int64_t)1 << 31);
   if (!pair) {
-    int rc = cin_quant_dual(dy, dy_dtype, M, N, sdm, 1, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, st,
-                            sstm, sstk, stream);
+    int rc = quant_dual(dy, dy_dtype, M, N, sdm, 1, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, st, sstm, sstk, pad,
+                        stream);
     if (rc != CIN_OK) return rc;
-    return cin_requant_row_to_block(xq, M, K, sxqm, xs, sxsm, sxsk, nullptr, 0, xbt, sxbtm, sblk, ssbm,
-                                    stream);
+    return requant(xq, M, K, sxqm, xs, sxsm, sxsk, nullptr, 0, xbt, sxbtm, sblk, ssbm, pad, stream);
   }
   const int dvec_t = aligned(qt, 16) && sqtm % 16 == 0 && tile_fits32(sqtm);
   const int rvec_t = aligned(xbt, 16) && sxbtm % 16 == 0 && tile_fits32(sxbtm);
@@ -2346,13 +2379,33 @@ int cin_quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64
 #define CIN_QBWD(DT)                                                                               \
   hipLaunchKernelGGL((k_quant_bwd<DT>), resident_grid<k_quant_bwd<DT>>(nt), kThreads, 0, stream_, dy, \
                      M, N, sdm, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, dvec_t, st, sstm, sstk, xq, K, \
-                     sxqm, xs, sxsm, sxsk, xbt, sxbtm, rvec_t, sblk, ssbm, nd, nt)
+                     sxqm, xs, sxsm, sxsk, xbt, sxbtm, rvec_t, sblk, ssbm, nd, nt, (int)pad)
   if (dy_dtype == CIN_DT_BF16)
     CIN_QBWD(CIN_DT_BF16);
   else
     CIN_QBWD(CIN_DT_F16);
 #undef CIN_QBWD
   return cin_check_launch("quant_backward");
+}
+
+int cin_quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm,
+                       int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                       uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk,
+                       const uint8_t* xq, int64_t K, int64_t sxqm, const float* xs, int64_t sxsm,
+                       int64_t sxsk, uint8_t* xbt, int64_t sxbtm, float* sblk, int64_t ssbm,
+                       void* stream) {
+  return quant_backward(dy, dy_dtype, M, N, sdm, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, st, sstm, sstk, xq, K,
+                        sxqm, xs, sxsm, sxsk, xbt, sxbtm, sblk, ssbm, false, stream);
+}
+
+int cin_quant_backward_padded(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm,
+                              int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                              uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk,
+                              const uint8_t* xq, int64_t K, int64_t sxqm, const float* xs, int64_t sxsm,
+                              int64_t sxsk, uint8_t* xbt, int64_t sxbtm, float* sblk, int64_t ssbm,
+                              void* stream) {
+  return quant_backward(dy, dy_dtype, M, N, sdm, round_scale, q, sqm, s, ssm, ssk, qt, sqtm, st, sstm, sstk, xq, K,
+                        sxqm, xs, sxsm, sxsk, xbt, sxbtm, sblk, ssbm, true, stream);
 }
 
 int cin_silu_mul_quant_rowwise(const void* h12, int in_dtype, int64_t M, int64_t H, int64_t s12,

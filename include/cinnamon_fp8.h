@@ -161,6 +161,19 @@ int cin_quant_backward(const void* dy, int dy_dtype, int64_t M, int64_t N, int64
                        void* stream);
 
 /*
+ * cin_quant_backward with the transposed outputs on whole 128-column tiles: qt [N, Mp] and
+ * xbt [K, Mp], Mp = 128 ceil(M / 128), zeros in the columns past M (row strides sqtm, sxbtm >=
+ * Mp).  The weight-gradient product then reduces over Mp: whole K blocks, aligned rows and
+ * full-line stores whatever the number of rows M, with the same sums.
+ */
+int cin_quant_backward_padded(const void* dy, int dy_dtype, int64_t M, int64_t N, int64_t sdm,
+                              int round_scale, uint8_t* q, int64_t sqm, float* s, int64_t ssm, int64_t ssk,
+                              uint8_t* qt, int64_t sqtm, float* st, int64_t sstm, int64_t sstk,
+                              const uint8_t* xq, int64_t K, int64_t sxqm, const float* xs, int64_t sxsm,
+                              int64_t sxsk, uint8_t* xbt, int64_t sxbtm, float* sblk, int64_t ssbm,
+                              void* stream);
+
+/*
  * Byte transpose: dst[c, r] = src[r, c] for an [R, C] matrix of codes.
  * Replaces the code-layout copies w_fp8.t().contiguous() (reference src/kernels.py:748).
  */

@@ -389,3 +389,26 @@ def test_e4m3_cast_exhaustive_through_rowwise(kern, dev, e):
         bad = (got != want).nonzero()
         assert bad.numel() == 0, f"binade {e} sign {sign}: {bad.numel()} codes differ, first x = {v[bad[0]].item()!r}"
         assert bool((q.view(torch.uint8)[:, 0] == 0x7E).all())
+
+
+# The padded form: one launch (whole column blocks), the two kernels with a masked edge block,
+# fp32, and rows no vector load takes (the row-wise passes); 1 row, a whole and a partial block
+@pytest.mark.parametrize("M,N,K,dtype", [
+    (1, 128, 256, torch.bfloat16), (127, 256, 128, torch.float16), (128, 128, 128, torch.bfloat16),
+    (1000, 384, 512, torch.bfloat16), (300, 200, 136, torch.bfloat16), (129, 256, 384, torch.float32),
+    (77, 131, 264, torch.bfloat16),
+])
+def test_backward_padded_equals_unpadded(kern, dev, M, N, K, dtype):
+    g = torch.Generator().manual_seed(M + N)
+    dy = (torch.randn(M, N, generator=g) * 1e-3).to(dtype).to(dev)
+    xq, xs = kern.quantize_fp8_rowwise(torch.randn(M, K, generator=g).to(dev), col_scales=True)
+    want = kern.quantize_fp8_backward(dy, xq, xs, True, col_scales=True)
+    got = kern._quant_bwd_padded_op(dy, xq, xs, True)
+    Mp = -(-M // 128) * 128
+    assert got[2].shape == (N, Mp) and got[4].shape == (K, Mp)
+    for a, b in zip(got, want):
+        a, b = (t.view(torch.uint8) if t.dtype == torch.float8_e4m3fn else t for t in (a, b))
+        if a.shape != b.shape:
+            assert torch.count_nonzero(a[:, M:]) == 0
+            a = a[:, :M]
+        assert torch.equal(a, b)
