@@ -396,7 +396,7 @@ def test_e4m3_cast_exhaustive_through_rowwise(kern, dev, e):
 @pytest.mark.parametrize("M,N,K,dtype", [
     (1, 128, 256, torch.bfloat16), (127, 256, 128, torch.float16), (128, 128, 128, torch.bfloat16),
     (1000, 384, 512, torch.bfloat16), (300, 200, 136, torch.bfloat16), (129, 256, 384, torch.float32),
-    (77, 131, 264, torch.bfloat16),
+    (77, 131, 264, torch.bfloat16), (16300, 128, 256, torch.bfloat16),
 ])
 def test_backward_padded_equals_unpadded(kern, dev, M, N, K, dtype):
     g = torch.Generator().manual_seed(M + N)
