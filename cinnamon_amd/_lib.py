@@ -127,7 +127,7 @@ def last_error() -> str:
 
 def call(name: str, *args) -> None:
     """Call an entry point; raise ValueError (bad argument) or RuntimeError on failure."""
-    rc = getattr(load(), name)(*args)
+    rc = getattr(_lib or load(), name)(*args)
     if rc != CIN_OK:
         msg = f"{name} failed ({rc}): {last_error()}"
         if rc == CIN_ERR_ARG:
@@ -144,10 +144,11 @@ def dtype_code(t) -> int:
         raise ValueError(f"unsupported dtype {dt}; expected bfloat16, float16 or float32") from None
 
 
-def stream_of(t: torch.Tensor) -> ctypes.c_void_p:
+def stream_of(t: torch.Tensor) -> int:
     """torch's current HIP stream on the tensor's device (as a hipStream_t)."""
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    # (the raw handle: torch.cuda.current_stream builds a Stream object, 2.2 us against 0.2)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
-def ptr(t: torch.Tensor | None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(0 if t is None else t.data_ptr())
+def ptr(t: torch.Tensor | None) -> int:
+    return 0 if t is None else t.data_ptr()

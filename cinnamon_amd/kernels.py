@@ -79,10 +79,16 @@ def custom_op(name: str, schema: str):
 
 def _plain_eager(*tensors) -> bool:
     """True outside tracing: no torch.compile, no dispatch mode (FakeTensor, make_fx,
-    functionalization), no functorch transform, and plain tensors."""
-    return (not torch.compiler.is_compiling() and _get_current_dispatch_mode() is None
-            and not torch._C._are_functorch_transforms_active()
-            and all(type(t) is torch.Tensor for t in tensors))
+    functionalization), no functorch transform, and plain tensors (or, where no graph is
+    recorded, parameters: the autograd Functions are handed the layers' own)."""
+    if (torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None
+            or torch._C._are_functorch_transforms_active()):
+        return False
+    for t in tensors:
+        c = type(t)
+        if c is not torch.Tensor and not (c is torch.nn.Parameter and not torch.is_grad_enabled()):
+            return False
+    return True
 
 
 def _run(op, *args):
@@ -90,7 +96,18 @@ def _run(op, *args):
     same kernels on the same arguments, without torch's dispatcher, whose host cost per call
     exceeds the device time of a small launch.  Only for operators without an autograd
     formula (these run inside the autograd Functions, or where no gradient is defined)."""
-    if _plain_eager(*(a for a in args if isinstance(a, torch.Tensor))):
+    if _plain_eager(*[a for a in args if isinstance(a, torch.Tensor)]):
+        return _LAUNCH[op](*args)
+    return op(*args)
+
+
+def _run_detached(op, *args):
+    """_run for an operator whose result could be mistaken for a differentiable one: with an
+    input that records a graph, the operator runs (and refuses the backward)."""
+    tensors = [a for a in args if isinstance(a, torch.Tensor)]
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return op(*args)
+    if _plain_eager(*tensors):
         return _LAUNCH[op](*args)
     return op(*args)
 
@@ -540,11 +557,14 @@ def _(x_fp8, scales, block_m, block_n):
 # Block-scaled FP8 GEMM (reference src/kernels.py:588-702)
 # ---------------------------------------------------------------------------
 def _kcontig(codes: torch.Tensor, K: int) -> tuple[torch.Tensor, int]:
-    """Return a [R, Kp] K-contiguous, 16-byte aligned uint8 view/copy and Kp (K padded to 16)."""
-    q = _codes_u8(codes)
+    """Return [R, Kp] K-contiguous, 16-byte aligned codes (themselves or a copy) and Kp (K padded to 16)."""
+    if codes.dtype != torch.float8_e4m3fn:
+        _codes_u8(codes)
     Kp = _cdiv(K, 16) * 16
-    if Kp == K and q.stride(1) == 1 and q.stride(0) % 16 == 0 and q.data_ptr() % 16 == 0:
-        return q, K
+    ld, unit = codes.stride()
+    if Kp == K and unit == 1 and ld % 16 == 0 and codes.data_ptr() % 16 == 0:
+        return codes, K  # (only its address and strides are used: codes are bytes in either dtype)
+    q = _codes_u8(codes)
     out = torch.zeros((q.shape[0], Kp), dtype=torch.uint8, device=q.device)
     out[:, :K].copy_(q)
     return out, Kp

@@ -11,8 +11,8 @@ from __future__ import annotations
 import torch
 
 from ._lib import call, dtype_code, ptr, stream_of
-from .kernels import (WeightCache, _cdiv, _codes_u8, _rows8, _kcontig, _require, _scale_buf, _scales_2d,
-                      _weight_cache_active, custom_op, quantize_fp8_blockwise_t,
+from .kernels import (WeightCache, _cdiv, _codes_u8, _rows8, _kcontig, _require, _run_detached, _scale_buf,
+                      _scales_2d, _weight_cache_active, custom_op, quantize_fp8_blockwise_t,
                       quantize_fp8_rowwise)
 
 
@@ -40,8 +40,8 @@ def fp8_grouped_gemm(a_codes: torch.Tensor, a_scales: torch.Tensor, w_codes: tor
     ends = expert_ends.to(torch.int64)
     _require(starts.numel() == E and ends.numel() == E, "expert ranges must have E entries")
     if out is None:
-        return _grouped_gemm_op(a_codes, a_scales, w_codes, w_scales, starts, ends, out_dtype,
-                                bool(zero_uncovered))
+        return _run_detached(_grouped_gemm_op, a_codes, a_scales, w_codes, w_scales, starts, ends, out_dtype,
+                             bool(zero_uncovered))
     _require(out.stride(1) == 1, "out must have unit column stride")
     return _grouped_gemm_into(a_codes, a_scales, w_codes, w_scales, starts, ends, out)
 
@@ -106,7 +106,7 @@ def quantize_fp8_dual_grouped(grad: torch.Tensor, expert_starts: torch.Tensor,
     _require(grad.is_cuda, "Input must be on CUDA")
     _require(grad.ndim == 2, "Input must be 2D")
     starts, ends = _ranges(expert_starts, expert_ends)
-    return _dual_grouped_op(grad, starts, ends, bool(round_scale), bool(col_scales))
+    return _run_detached(_dual_grouped_op, grad, starts, ends, bool(round_scale), bool(col_scales))
 
 
 @custom_op("quant_dual_grouped",
@@ -148,7 +148,7 @@ def requantize_grouped_t(x_fp8: torch.Tensor, x_scale: torch.Tensor, expert_star
     _require(x_fp8.is_cuda, "Input must be on CUDA")
     _codes_u8(x_fp8)
     starts, ends = _ranges(expert_starts, expert_ends)
-    return _requant_grouped_op(x_fp8, x_scale, starts, ends)
+    return _run_detached(_requant_grouped_op, x_fp8, x_scale, starts, ends)
 
 
 @custom_op("requant_row_to_block_grouped",
@@ -185,7 +185,7 @@ def fp8_grouped_wgrad(g_t: torch.Tensor, g_st: torch.Tensor, x_bt: torch.Tensor,
     _require(g_t.is_cuda and x_bt.is_cuda, "Input must be on CUDA")
     starts, ends = _ranges(expert_starts, expert_ends)
     _require(x_bt.shape[1] == g_t.shape[1], "operands must share the padded token axis")
-    return _grouped_wgrad_op(g_t, g_st, x_bt, x_blk, starts, ends, int(num_tokens), out_dtype)
+    return _run_detached(_grouped_wgrad_op, g_t, g_st, x_bt, x_blk, starts, ends, int(num_tokens), out_dtype)
 
 
 @custom_op("grouped_wgrad_fp8", "(Tensor g_t, Tensor g_st, Tensor x_bt, Tensor x_blk, Tensor starts, "
@@ -227,8 +227,8 @@ def fp8_grouped_dgrad(g_fp8: torch.Tensor, g_scale: torch.Tensor, w_codes_t: tor
     _require(N == n_out_per_expert and EN == E * N and N % 128 == 0,
              "w_codes_t must be [K, E*N] with N a multiple of 128")
     if out is None:
-        return _grouped_dgrad_op(g_fp8, g_scale, w_codes_t, w_scales, starts, ends, out_dtype,
-                                 bool(zero_uncovered))
+        return _run_detached(_grouped_dgrad_op, g_fp8, g_scale, w_codes_t, w_scales, starts, ends, out_dtype,
+                             bool(zero_uncovered))
     return _grouped_dgrad_into(g_fp8, g_scale, w_codes_t, w_scales, starts, ends, out)
 
 
@@ -279,7 +279,7 @@ def silu_mul_quantize_fp8(h12: torch.Tensor, out_dtype: torch.dtype | None = Non
     Returns (codes float8_e4m3fn [M, H], scales fp32 [M, ceil(H/128)])."""
     _require(h12.is_cuda, "Input must be on CUDA")
     _require(h12.ndim == 2 and h12.shape[1] % 2 == 0, "h12 must be [M, 2H]")
-    return _silu_mul_quant_op(h12, out_dtype or h12.dtype, bool(round_scale), bool(col_scales))
+    return _run_detached(_silu_mul_quant_op, h12, out_dtype or h12.dtype, bool(round_scale), bool(col_scales))
 
 
 @custom_op("silu_mul_quant_rowwise",
@@ -308,7 +308,7 @@ def swiglu_backward(dh: torch.Tensor, h12: torch.Tensor) -> torch.Tensor:
     _require(dh.is_cuda and h12.is_cuda, "Input must be on CUDA")
     M, H = dh.shape
     _require(h12.shape == (M, 2 * H), "h12 must be [M, 2H]")
-    return _swiglu_backward_op(dh, h12)
+    return _run_detached(_swiglu_backward_op, dh, h12)
 
 
 @custom_op("swiglu_backward", "(Tensor dh, Tensor h12) -> Tensor")
@@ -339,9 +339,9 @@ def swiglu_backward_dual_grouped(dh: torch.Tensor, h12: torch.Tensor, expert_sta
     _require(h12.shape == (T, 2 * H), "h12 must be [T, 2H]")
     starts, ends = _ranges(expert_starts, expert_ends)
     if H % 128 != 0:
-        return _dual_grouped_op(_swiglu_backward_op(dh, h12), starts, ends, bool(round_scale),
-                                bool(col_scales))
-    return _swiglu_dual_grouped_op(dh, h12, starts, ends, bool(round_scale), bool(col_scales))
+        return _run_detached(_dual_grouped_op, _run_detached(_swiglu_backward_op, dh, h12), starts, ends,
+                             bool(round_scale), bool(col_scales))
+    return _run_detached(_swiglu_dual_grouped_op, dh, h12, starts, ends, bool(round_scale), bool(col_scales))
 
 
 @custom_op("swiglu_dual_grouped",

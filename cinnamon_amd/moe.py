@@ -23,7 +23,7 @@ import torch
 
 from . import layers
 from ._lib import call, dtype_code, ptr, stream_of
-from .kernels import _cdiv, _require, _scale_buf, custom_op
+from .kernels import _cdiv, _require, _run_detached, _scale_buf, custom_op
 
 _ROUTE_CHUNK = 1024  # assignments per route workgroup (csrc/moe.hip kChunk)
 MAX_EXPERTS = 4096
@@ -47,7 +47,7 @@ def moe_route(top_idx: torch.Tensor, n_experts: int):
     _require(top_idx.is_cuda, "Input must be on CUDA")
     _require(top_idx.ndim == 2, "top_idx must be [n_tokens, top_k]")
     _require(1 <= n_experts <= MAX_EXPERTS, f"n_experts must be in [1, {MAX_EXPERTS}]")
-    return _route_op(top_idx.to(torch.int64).contiguous(), int(n_experts))
+    return _run_detached(_route_op, top_idx.to(torch.int64).contiguous(), int(n_experts))
 
 
 @custom_op("moe_route", "(Tensor idx, int n_experts) -> (Tensor, Tensor, Tensor, Tensor, Tensor)")
@@ -91,9 +91,9 @@ def moe_gather_quantize(x: torch.Tensor, perm: torch.Tensor, top_k: int, round_s
     _require(top_k >= 1, "top_k must be >= 1")
     if inv is not None:
         _require(inv.numel() == x.shape[0] * top_k, "inv must hold n_tokens * top_k entries")
-        return _scatter_quant_op(x, perm.to(torch.int64), inv.to(torch.int32), int(top_k),
-                                 bool(round_scale), bool(col_scales))
-    return _gather_quant_op(x, perm.to(torch.int64), int(top_k), bool(round_scale), bool(col_scales))
+        return _run_detached(_scatter_quant_op, x, perm.to(torch.int64), inv.to(torch.int32), int(top_k),
+                             bool(round_scale), bool(col_scales))
+    return _run_detached(_gather_quant_op, x, perm.to(torch.int64), int(top_k), bool(round_scale), bool(col_scales))
 
 
 def _codes_rows8(A, D, like):
@@ -176,7 +176,7 @@ def moe_gather_sum(g: torch.Tensor, inv: torch.Tensor, top_k: int,
     _require(g.is_cuda and inv.is_cuda, "Input must be on CUDA")
     _require(1 <= top_k <= MAX_TOP_K, f"top_k must be in [1, {MAX_TOP_K}]")
     _require(inv.numel() % top_k == 0, "inv must hold n_tokens * top_k entries")
-    return _gather_sum_op(g, inv.to(torch.int32), int(top_k), out_dtype)
+    return _run_detached(_gather_sum_op, g, inv.to(torch.int32), int(top_k), out_dtype)
 
 
 @custom_op("moe_gather_sum", "(Tensor g, Tensor inv, int top_k, ScalarType out_dtype) -> Tensor")
@@ -209,7 +209,7 @@ def moe_combine(sorted_out: torch.Tensor, top_scores: torch.Tensor, inv: torch.T
     _require(inv.numel() == top_scores.numel(), "inv must hold n_tokens * top_k entries")
     _require(sorted_out.dtype in (torch.float32, torch.float16, torch.bfloat16),
              "sorted_out must be fp32, fp16 or bf16 (the experts' output)")
-    return _combine_op(sorted_out, top_scores, inv.to(torch.int32))
+    return _run_detached(_combine_op, sorted_out, top_scores, inv.to(torch.int32))
 
 
 @custom_op("moe_combine", "(Tensor y, Tensor scores, Tensor inv) -> Tensor")
@@ -244,8 +244,8 @@ def moe_combine_backward(dout: torch.Tensor, sorted_out: torch.Tensor, top_score
     if dy_dtype is None:
         dy_dtype = sorted_out.dtype
     _require(dy_dtype in (torch.float32, torch.bfloat16, torch.float16), "dy_dtype must be fp32, bf16 or fp16")
-    return _combine_bwd_op(dout.float(), sorted_out, top_scores, perm.to(torch.int64),
-                           inv.to(torch.int32), dy_dtype)
+    return _run_detached(_combine_bwd_op, dout.float(), sorted_out, top_scores, perm.to(torch.int64),
+                         inv.to(torch.int32), dy_dtype)
 
 
 @custom_op("moe_combine_backward",

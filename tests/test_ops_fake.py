@@ -241,3 +241,23 @@ def test_eager_calls_bypass_the_dispatcher_only_outside_tracing():
     assert seen == [False]
     assert all(op in kernels._LAUNCH for op in (kernels._quant_fwd_op, kernels._gemm_bs_op,
                                                  kernels._quant_bwd_op, kernels._quant_rowwise_op))
+
+
+def test_direct_launch_only_where_no_graph_is_recorded(monkeypatch):
+    """kernels._run_detached launches directly unless an input records a graph (the operator
+    then refuses the backward); a parameter counts as a plain tensor only under no_grad."""
+    took = []
+
+    def op(*args):
+        took.append("operator")
+
+    monkeypatch.setitem(kernels._LAUNCH, op, lambda *args: took.append("launch"))
+    plain, leaf, param = torch.zeros(2), torch.zeros(2, requires_grad=True), torch.nn.Parameter(torch.zeros(2))
+    kernels._run_detached(op, plain, 3)
+    kernels._run_detached(op, plain, leaf)
+    kernels._run_detached(op, param)
+    kernels._run(op, param)
+    with torch.no_grad():
+        kernels._run_detached(op, plain, leaf, param)
+        kernels._run(op, param)
+    assert took == ["launch", "operator", "operator", "operator", "launch", "launch"]
