@@ -18,6 +18,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include <mutex>
 
 #include "cin_common.h"
@@ -235,13 +237,15 @@ __global__ __launch_bounds__(64) void k_route_scatter(const int64_t* __restrict_
 
 // Sorted positions of token t's assignments in increasing order, with their slots; the
 // missing ones (dropped ids, slots past k) get INT32_MAX and sort last.  A fixed
-// compare-swap network keeps every index a compile-time one (registers, no scratch).
+// compare-swap network keeps every index a compile-time one (registers, no scratch).  KM: a
+// compile-time bound on k (see with_k).
 // Returns the number of valid positions.
+template <int KM>
 __device__ inline int token_positions(const int32_t* __restrict__ inv, int64_t t, int k, int64_t A,
-                                      int32_t (&pos)[kMaxTopK], int32_t (&slot)[kMaxTopK]) {
+                                      int32_t (&pos)[KM], int32_t (&slot)[KM]) {
   int n = 0;
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) {
+  for (int j = 0; j < KM; ++j) {
     const int32_t p = j < k ? inv[t * k + j] : -1;
     const bool ok = p >= 0 && p < A;
     pos[j] = ok ? p : INT32_MAX;
@@ -249,9 +253,9 @@ __device__ inline int token_positions(const int32_t* __restrict__ inv, int64_t t
     n += ok;
   }
 #pragma unroll
-  for (int i = 0; i < kMaxTopK - 1; ++i) {
+  for (int i = 0; i < KM - 1; ++i) {
 #pragma unroll
-    for (int j = 0; j < kMaxTopK - 1 - i; ++j) {
+    for (int j = 0; j < KM - 1 - i; ++j) {
       if (pos[j] > pos[j + 1]) {
         const int32_t tp = pos[j], ts = slot[j];
         pos[j] = pos[j + 1];
@@ -317,20 +321,20 @@ __device__ __forceinline__ float piece_elem(const uint4 (&q)[W], int e) {
   }
 }
 
-// W 16-byte pieces of G of a token's rows, pos[j0] .. pos[j0 + G - 1], at byte `cb` of
-// each row (rows `rb` bytes apart), every load issued before any result is used: one wave
-// keeps G W loads in flight instead of one.  Rows at or past n load row pos[j0] again
+// W 16-byte pieces, PS pieces apart, of G of a token's rows, pos[j0] .. pos[j0 + G - 1], at byte
+// `cb` of each row (rows `rb` bytes apart), every load issued before any result is used: one
+// wave keeps G W loads in flight instead of one.  Rows at or past n load row pos[j0] again
 // (j0 < n); their pieces are never used.  Needs 16-byte aligned pieces.
-template <int G, int W>
+template <int G, int W, int PS, int KM>
 __device__ __forceinline__ void load_rows(const void* base, int64_t cb, int64_t rb,
-                                          const int32_t (&pos)[kMaxTopK], int j0, int n,
+                                          const int32_t (&pos)[KM], int j0, int n,
                                           uint4 (&raw)[G][W]) {
 #pragma unroll
   for (int jj = 0; jj < G; ++jj) {
     const int64_t r = j0 + jj < n ? pos[j0 + jj] : pos[j0];
     const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(base) + r * rb + cb);
 #pragma unroll
-    for (int u = 0; u < W; ++u) raw[jj][u] = p[u];
+    for (int u = 0; u < W; ++u) raw[jj][u] = p[u * PS];
   }
 }
 
@@ -357,188 +361,130 @@ __device__ inline void store4(void* base, int64_t off, int64_t nv, const float (
   }
 }
 
-// dx[t] = sum of g[r] over token t's sorted positions r (increasing r), fp32 sums.
-// One wave per token; lane l covers columns 8 l + 512 i of fp32 rows and 16 l + 1024 i of
-// 16-bit rows (two 16-byte pieces per row and step: the rows sit at scattered sorted
-// positions, and 2 KB runs per row read ~6-10% faster than 1 KB runs).
-template <int GT, int OT>
-__global__ __launch_bounds__(kRT) void k_moe_gather_sum(const void* __restrict__ g, int64_t sgm,
-                                                        const int32_t* __restrict__ inv,
-                                                        int64_t T, int k, int64_t A, int64_t N,
-                                                        void* __restrict__ out, int64_t som) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = ((int64_t)blockIdx.x * kRT + threadIdx.x) >> 6;
-  if (t >= T) return;  // uniform per wave
-  int32_t pos[kMaxTopK], slot[kMaxTopK];
-  const int n = token_positions(inv, t, k, A, pos, slot);
-  // whole chunks of rows whose pieces are 16-byte aligned take the batched loads
-  const bool vec = ((((uintptr_t)g) & 15) == 0) && ((sgm * (GT == CIN_DT_F32 ? 4 : 2)) & 15) == 0;
-  if constexpr (GT == CIN_DT_F32) {
-    for (int64_t c = (int64_t)lane * 8; c < N; c += 512) {
-      float acc[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-      if (vec && c + 8 <= N) {
-#pragma unroll
-        for (int j0 = 0; j0 < kMaxTopK; j0 += kRowBatch) {
-          if (j0 < n) {
-            uint4 raw[kRowBatch][2];
-            load_rows<kRowBatch, 2>(g, c * 4, sgm * 4, pos, j0, n, raw);
-#pragma unroll
-            for (int jj = 0; jj < kRowBatch; ++jj)
-              if (j0 + jj < n)
-                for (int e = 0; e < 8; ++e) acc[e >> 2][e & 3] = acc[e >> 2][e & 3] + piece_elem<GT, 2>(raw[jj], e);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kMaxTopK; ++j) {
-          if (j < n) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              float v[4];
-              load4<GT>(g, (int64_t)pos[j] * sgm + c + 4 * u, N - c - 4 * u, v);
-              for (int e = 0; e < 4; ++e) acc[u][e] = acc[u][e] + v[e];
-            }
-          }
-        }
-      }
-      store4<OT>(out, t * som + c, N - c, acc[0]);
-      store4<OT>(out, t * som + c + 4, N - c - 4, acc[1]);
+// One 16-byte piece's worth of columns: 4 of fp32 rows, 8 of 16-bit rows.
+template <int DT>
+constexpr int kPiece = DT == CIN_DT_F32 ? 4 : 8;
+
+template <int DT>
+__device__ __forceinline__ void load_piece(const void* base, int64_t off, int64_t nv, float (&v)[kPiece<DT>]) {
+  if constexpr (DT == CIN_DT_F32)
+    load4<DT>(base, off, nv, v);
+  else
+    load8h<DT>(base, off, nv, v);
+}
+
+template <int OT, int E>
+__device__ __forceinline__ void store_piece(void* base, int64_t off, int64_t nv, const float (&v)[E]) {
+  if constexpr (E == 8 && OT != CIN_DT_F32) {
+    uint16_t* p = static_cast<uint16_t*>(base) + off;
+    if (nv >= 8 && (((uintptr_t)p) & 15) == 0) {
+      *reinterpret_cast<uint4*>(p) = make_uint4(f32x2_to_half2_bits<OT>(v[0], v[1]), f32x2_to_half2_bits<OT>(v[2], v[3]),
+                                                f32x2_to_half2_bits<OT>(v[4], v[5]), f32x2_to_half2_bits<OT>(v[6], v[7]));
+      return;
     }
-  } else {
-    // 16-bit rows: 16 columns per lane (two 16-byte loads), 2 KB runs per row
-    for (int64_t c = (int64_t)lane * 16; c < N; c += 1024) {
-      float acc[16];
+  }
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-      if (vec && c + 16 <= N) {
-#pragma unroll
-        for (int j0 = 0; j0 < kMaxTopK; j0 += kRowBatch) {
-          if (j0 < n) {
-            uint4 raw[kRowBatch][2];
-            load_rows<kRowBatch, 2>(g, c * 2, sgm * 2, pos, j0, n, raw);
-#pragma unroll
-            for (int jj = 0; jj < kRowBatch; ++jj)
-              if (j0 + jj < n)
-                for (int e = 0; e < 16; ++e) acc[e] = acc[e] + piece_elem<GT, 2>(raw[jj], e);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kMaxTopK; ++j) {
-          if (j < n) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              float v[8];
-              load8h<GT>(g, (int64_t)pos[j] * sgm + c + 8 * u, N - c - 8 * u, v);
-              for (int e = 0; e < 8; ++e) acc[8 * u + e] = acc[8 * u + e] + v[e];
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float a4[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-        store4<OT>(out, t * som + c + 4 * q, N - c - 4 * q, a4);
-      }
-    }
+  for (int q = 0; q < E / 4; ++q) {
+    const float a[4] = {v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+    store4<OT>(base, off + 4 * q, nv - 4 * q, a);
   }
 }
 
-template <int ST>
-__device__ inline float score_at(const void* s, int64_t off) {
-  return load_elem(s, ST, off);
+// Sum over a token's sorted positions r (increasing) of its row pieces, each times w[j] if
+// WEIGHTED (a product then an add, both rounded: built without contraction), in fp32, into
+// out's row t: the combine and the gather sum.
+// nch waves per token, one per step of 128 pieces (or every nch-th).  In a step a lane holds
+// pieces l and l + 64: 2 KB runs of the scattered rows, and stores that run along the lanes
+// (with both pieces of a lane side by side, an fp32 output left in 16-byte stores 64 bytes
+// apart).  The work per wave grows with KM, the bound on k, not with the largest k: sorting 16
+// positions and loading 8 rows for k = 2 held the wave to 2 per SIMD.  Combine / gather sum in
+// us, before and after: 16384 tokens, k 2, 1024 fp16 columns, 55.5 / 39.4 and 29.9 / 17.0 (4.5 and
+// 5.9 TB/s); 16384, k 8, 7168, 520 / 433 and 427 / 402; 64, k 8, 7168, 22.8 / 16.9 and 11.0 / 10.2.
+template <int GT, int OT, int KM, bool WEIGHTED>
+__device__ __forceinline__ void sum_rows(const void* __restrict__ g, int64_t sgm, const int32_t (&pos)[KM], int n,
+                                         const float (&w)[KM], int64_t t, int ch, int nch, int64_t N,
+                                         void* __restrict__ out, int64_t som) {
+  constexpr int RB = KM < kRowBatch ? KM : kRowBatch;
+  constexpr int E = kPiece<GT>, ES = GT == CIN_DT_F32 ? 4 : 2;
+  const int lane = threadIdx.x & 63;
+  // whole steps of rows whose pieces are 16-byte aligned take the batched loads
+  const bool vec = ((((uintptr_t)g) & 15) == 0) && ((sgm * ES) & 15) == 0;
+  for (int64_t c = (int64_t)(ch * 128 + lane) * E; c < N; c += (int64_t)nch * 128 * E) {
+    float acc[2][E];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int e = 0; e < E; ++e) acc[u][e] = 0.0f;
+    if (vec && c + 65 * E <= N) {
+#pragma unroll
+      for (int j0 = 0; j0 < KM; j0 += RB) {
+        if (j0 < n) {
+          uint4 raw[RB][2];
+          load_rows<RB, 2, 64>(g, c * ES, sgm * ES, pos, j0, n, raw);
+#pragma unroll
+          for (int jj = 0; jj < RB; ++jj)
+            if (j0 + jj < n)
+#pragma unroll
+              for (int u = 0; u < 2; ++u) {
+                const uint4 piece[1] = {raw[jj][u]};
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                  const float v = piece_elem<GT, 1>(piece, e);
+                  acc[u][e] = acc[u][e] + (WEIGHTED ? v * w[j0 + jj] : v);
+                }
+              }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < KM; ++j) {
+        if (j < n) {
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            float v[E];
+            load_piece<GT>(g, (int64_t)pos[j] * sgm + c + 64 * E * u, N - c - 64 * E * u, v);
+#pragma unroll
+            for (int e = 0; e < E; ++e) acc[u][e] = acc[u][e] + (WEIGHTED ? v[e] * w[j] : v[e]);
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) store_piece<OT, E>(out, t * som + c + 64 * E * u, N - c - 64 * E * u, acc[u]);
+  }
 }
 
-// out[t] = sum over the token's positions r (increasing) of y[r] * score[t, slot(r)]:
-// a product then an add, both rounded (built without contraction), fp32.  One wave per
-// token; lane l covers columns 8 l + 512 i of fp32 rows (as k_moe_gather_sum) and
-// 16 l + 1024 i of 16-bit rows: 2 KB runs per scattered row either way.
-template <int YT, int ST>
+// dx[t] = sum of g[r] over token t's sorted positions r (increasing r), fp32 sums.
+template <int GT, int OT, int KM>
+__global__ __launch_bounds__(kRT) void k_moe_gather_sum(const void* __restrict__ g, int64_t sgm,
+                                                        const int32_t* __restrict__ inv,
+                                                        int64_t T, int k, int64_t A, int64_t N,
+                                                        void* __restrict__ out, int64_t som, int nch) {
+  const int64_t wave = ((int64_t)blockIdx.x * kRT + threadIdx.x) >> 6;
+  const int64_t t = wave / nch;
+  if (t >= T) return;  // uniform per wave
+  int32_t pos[KM], slot[KM];
+  const int n = token_positions(inv, t, k, A, pos, slot);
+  const float w[KM] = {};
+  sum_rows<GT, OT, KM, false>(g, sgm, pos, n, w, t, (int)(wave - t * nch), nch, N, out, som);
+}
+
+// out[t] = sum over the token's positions r (increasing) of y[r] * score[t, slot(r)], fp32.
+template <int YT, int ST, int KM>
 __global__ __launch_bounds__(kRT) void k_moe_combine(const void* __restrict__ y, int64_t sym,
                                                      const void* __restrict__ scores,
                                                      int64_t ssm, const int32_t* __restrict__ inv,
                                                      int64_t T, int k, int64_t A, int64_t N,
-                                                     float* __restrict__ out, int64_t som) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = ((int64_t)blockIdx.x * kRT + threadIdx.x) >> 6;
+                                                     float* __restrict__ out, int64_t som, int nch) {
+  const int64_t wave = ((int64_t)blockIdx.x * kRT + threadIdx.x) >> 6;
+  const int64_t t = wave / nch;
   if (t >= T) return;  // uniform per wave
-  int32_t pos[kMaxTopK], slot[kMaxTopK];
+  int32_t pos[KM], slot[KM];
   const int n = token_positions(inv, t, k, A, pos, slot);
-  float w[kMaxTopK];
+  float w[KM];
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) w[j] = j < n ? score_at<ST>(scores, t * ssm + slot[j]) : 0.0f;
-  // whole chunks of rows whose pieces are 16-byte aligned take the batched loads
-  const bool vec = ((((uintptr_t)y) & 15) == 0) && ((sym * (YT == CIN_DT_F32 ? 4 : 2)) & 15) == 0;
-  if constexpr (YT == CIN_DT_F32) {
-    for (int64_t c = (int64_t)lane * 8; c < N; c += 512) {
-      float acc[2][4] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
-      if (vec && c + 8 <= N) {
-#pragma unroll
-        for (int j0 = 0; j0 < kMaxTopK; j0 += kRowBatch) {
-          if (j0 < n) {
-            uint4 raw[kRowBatch][2];
-            load_rows<kRowBatch, 2>(y, c * 4, sym * 4, pos, j0, n, raw);
-#pragma unroll
-            for (int jj = 0; jj < kRowBatch; ++jj)
-              if (j0 + jj < n)
-                for (int e = 0; e < 8; ++e)
-                  acc[e >> 2][e & 3] = acc[e >> 2][e & 3] + piece_elem<YT, 2>(raw[jj], e) * w[j0 + jj];
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kMaxTopK; ++j) {
-          if (j < n) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              float v[4];
-              load4<YT>(y, (int64_t)pos[j] * sym + c + 4 * u, N - c - 4 * u, v);
-              for (int e = 0; e < 4; ++e) acc[u][e] = acc[u][e] + v[e] * w[j];
-            }
-          }
-        }
-      }
-      store4<CIN_DT_F32>(out, t * som + c, N - c, acc[0]);
-      store4<CIN_DT_F32>(out, t * som + c + 4, N - c - 4, acc[1]);
-    }
-  } else {
-    // 16-bit rows: 16 columns per lane (two 16-byte loads), the same 2 KB runs per row
-    for (int64_t c = (int64_t)lane * 16; c < N; c += 1024) {
-      float acc[16];
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-      if (vec && c + 16 <= N) {
-#pragma unroll
-        for (int j0 = 0; j0 < kMaxTopK; j0 += kRowBatch) {
-          if (j0 < n) {
-            uint4 raw[kRowBatch][2];
-            load_rows<kRowBatch, 2>(y, c * 2, sym * 2, pos, j0, n, raw);
-#pragma unroll
-            for (int jj = 0; jj < kRowBatch; ++jj)
-              if (j0 + jj < n)
-                for (int e = 0; e < 16; ++e) acc[e] = acc[e] + piece_elem<YT, 2>(raw[jj], e) * w[j0 + jj];
-          }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < kMaxTopK; ++j) {
-          if (j < n) {
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-              float v[8];
-              load8h<YT>(y, (int64_t)pos[j] * sym + c + 8 * u, N - c - 8 * u, v);
-              for (int e = 0; e < 8; ++e) acc[8 * u + e] = acc[8 * u + e] + v[e] * w[j];
-            }
-          }
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float a4[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-        store4<CIN_DT_F32>(out, t * som + c + 4 * q, N - c - 4 * q, a4);
-      }
-    }
-  }
+  for (int j = 0; j < KM; ++j) w[j] = j < n ? load_elem(scores, ST, t * ssm + slot[j]) : 0.0f;
+  sum_rows<YT, CIN_DT_F32, KM, true>(y, sym, pos, n, w, t, (int)(wave - t * nch), nch, N, out, som);
 }
 
 // Combine backward, both gradients in one pass per token (one wave): the token's dout row
@@ -546,8 +492,10 @@ __global__ __launch_bounds__(kRT) void k_moe_combine(const void* __restrict__ y,
 // gradient dscore[t, j] = sum_c dout[t, c] * y[r, c] (lane l over columns 8 l + 512 i, then
 // a wave sum) and dy[r] = dout[t] * score[t, j] is written in dy's dtype DT (RNE of the
 // fp32 product).  Slots whose assignment was dropped get dscore 0; the dy rows no
-// assignment maps to are zeroed by k_moe_zero_unmapped_rows.
-template <int YT, int DT>
+// assignment maps to are zeroed by k_moe_zero_unmapped_rows.  Bound by its reads and writes;
+// with the bound on k compiled in, 16384 tokens, k 2, 1024 columns 86.8 -> 39.9 us (5.1 TB/s), k 8,
+// 7168 columns as before (856 us, 4.9 TB/s).
+template <int YT, int DT, int KM>
 __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
     const float* __restrict__ dout, int64_t sdm, const void* __restrict__ y, int64_t sym,
     const void* __restrict__ scores, int st, int64_t ssm, const int32_t* __restrict__ inv, int64_t T,
@@ -555,16 +503,17 @@ __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
   const int lane = threadIdx.x & 63;
   const int64_t t = ((int64_t)blockIdx.x * kRT + threadIdx.x) >> 6;
   if (t >= T) return;  // uniform per wave
-  int32_t pos[kMaxTopK], slot[kMaxTopK];
+  constexpr int RB = KM < kRowBatch ? KM : kRowBatch;
+  int32_t pos[KM], slot[KM];
   const int n = token_positions(inv, t, k, A, pos, slot);
-  float w[kMaxTopK], acc[kMaxTopK];
+  float w[KM], acc[KM];
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) {
+  for (int j = 0; j < KM; ++j) {
     w[j] = j < n ? load_elem(scores, st, t * ssm + slot[j]) : 0.0f;
     acc[j] = 0.0f;
   }
   const int64_t db = t * sdm;
-  // 16-bit rows whose 16-byte pieces are aligned: up to kRowBatch rows' pieces are loaded
+  // 16-bit rows whose 16-byte pieces are aligned: up to RB rows' pieces are loaded
   // together before any is used (the per-row form has one row's load in flight per wave);
   // the same products and sums in the same order either way
   const bool vec = YT != CIN_DT_F32 && ((((uintptr_t)y) & 15) == 0) && (((sym * 2) & 15) == 0);
@@ -575,23 +524,18 @@ __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
     if constexpr (YT != CIN_DT_F32) {
       if (vec && c + 8 <= N) {
 #pragma unroll
-        for (int j0 = 0; j0 < kMaxTopK; j0 += kRowBatch) {
+        for (int j0 = 0; j0 < KM; j0 += RB) {
           if (j0 < n) {
-            uint4 raw[kRowBatch][1];
-            load_rows<kRowBatch, 1>(y, c * 2, sym * 2, pos, j0, n, raw);
+            uint4 raw[RB][1];
+            load_rows<RB, 1, 1>(y, c * 2, sym * 2, pos, j0, n, raw);
 #pragma unroll
-            for (int jj = 0; jj < kRowBatch; ++jj) {
+            for (int jj = 0; jj < RB; ++jj) {
               const int j = j0 + jj;
               if (j < n) {
                 for (int e = 0; e < 8; ++e) acc[j] += a[e >> 2][e & 3] * piece_elem<YT, 1>(raw[jj], e);
-                float d0[4], d1[4];
-                for (int e = 0; e < 4; ++e) {
-                  d0[e] = a[0][e] * w[j];
-                  d1[e] = a[1][e] * w[j];
-                }
-                const int64_t ob = (int64_t)pos[j] * sdym;
-                store4<DT>(dy, ob + c, N - c, d0);
-                store4<DT>(dy, ob + c + 4, N - c - 4, d1);
+                float d[8];
+                for (int e = 0; e < 8; ++e) d[e] = a[e >> 2][e & 3] * w[j];
+                store_piece<DT, 8>(dy, (int64_t)pos[j] * sdym + c, N - c, d);
               }
             }
           }
@@ -600,7 +544,7 @@ __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
       }
     }
 #pragma unroll
-    for (int j = 0; j < kMaxTopK; ++j) {
+    for (int j = 0; j < KM; ++j) {
       if (j < n) {
         const int64_t yb = (int64_t)pos[j] * sym;
         float b[8];
@@ -628,7 +572,7 @@ __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
     }
   }
 #pragma unroll
-  for (int j = 0; j < kMaxTopK; ++j) {
+  for (int j = 0; j < KM; ++j) {
     if (j < n) {
       const float sum = wave_sum(acc[j]);
       if (lane == 0) dscores[t * k + slot[j]] = sum;
@@ -654,6 +598,28 @@ __global__ __launch_bounds__(kRT) void k_moe_zero_unmapped_rows(const int64_t* _
   if (i >= 0 && i < T * k) return;  // uniform per wave
   const float z[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int64_t c = (int64_t)lane * 4; c < N; c += 256) store4<DT>(dy, r * sdym + c, N - c, z);
+}
+
+// launch(integral_constant KM), the smallest compiled bound on k: registers, row loads and the
+// sort of a token's positions all grow with the bound.
+template <class F>
+void with_k(int64_t k, F launch) {
+  if (k <= 2)
+    launch(std::integral_constant<int, 2>{});
+  else if (k <= 4)
+    launch(std::integral_constant<int, 4>{});
+  else if (k <= 8)
+    launch(std::integral_constant<int, 8>{});
+  else
+    launch(std::integral_constant<int, kMaxTopK>{});
+}
+
+// Waves per token of the combine and the gather sum: one per step of 128 16-byte pieces (one
+// in all where the grid could not hold them).  16384 tokens, k 8, 7168 columns: 466 and 395 us,
+// with one wave a token 515 and 433.
+int token_waves(int64_t T, int64_t N, int dtype) {
+  const int64_t steps = cdiv(N, dtype == CIN_DT_F32 ? 512 : 1024);
+  return steps < (1 << 30) && cdiv(T * steps * 64, kRT) < ((int64_t)1 << 31) ? (int)steps : 1;
 }
 
 // The route's three launches over a caller's int32 workspace of ws_elems entries.
@@ -755,10 +721,14 @@ int cin_moe_gather_sum(const void* g, int g_dtype, int64_t sgm, const int32_t* i
   if (T == 0 || N == 0) return CIN_OK;
   CIN_CHECK_ARG(g && inv && out && sgm >= N && som >= N, "moe_gather_sum: bad pointers or strides");
   CIN_CHECK_ARG(cdiv(T * 64, kRT) < ((int64_t)1 << 31), "moe_gather_sum: grid too large");
-  const unsigned grid = (unsigned)cdiv(T * 64, kRT);  // one wave per token
+  const int nch = token_waves(T, N, g_dtype);
+  const unsigned grid = (unsigned)cdiv(T * nch * 64, kRT);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CIN_GS(GT, OT) \
-  hipLaunchKernelGGL((k_moe_gather_sum<GT, OT>), grid, kRT, 0, s, g, sgm, inv, T, (int)k, A, N, out, som)
+#define CIN_GS(GT, OT)                                                                                         \
+  with_k(k, [&](auto km) {                                                                                     \
+    hipLaunchKernelGGL((k_moe_gather_sum<GT, OT, decltype(km)::value>), grid, kRT, 0, s, g, sgm, inv, T, (int)k, A, \
+                       N, out, som, nch);                                                                      \
+  })
   if (g_dtype == CIN_DT_F32) {
     if (out_dtype == CIN_DT_F32) CIN_GS(CIN_DT_F32, CIN_DT_F32);
     else if (out_dtype == CIN_DT_BF16) CIN_GS(CIN_DT_F32, CIN_DT_BF16);
@@ -787,10 +757,14 @@ int cin_moe_combine(const void* y, int y_dtype, int64_t sym, const void* scores,
   CIN_CHECK_ARG(y && scores && inv && out && sym >= N && som >= N && ssm >= k,
                 "moe_combine: bad pointers or strides");
   CIN_CHECK_ARG(cdiv(T * 64, kRT) < ((int64_t)1 << 31), "moe_combine: grid too large");
-  const unsigned grid = (unsigned)cdiv(T * 64, kRT);  // one wave per token
+  const int nch = token_waves(T, N, y_dtype);
+  const unsigned grid = (unsigned)cdiv(T * nch * 64, kRT);
   hipStream_t s = static_cast<hipStream_t>(stream);
-#define CIN_COMB(YT, ST) \
-  hipLaunchKernelGGL((k_moe_combine<YT, ST>), grid, kRT, 0, s, y, sym, scores, ssm, inv, T, (int)k, A, N, out, som)
+#define CIN_COMB(YT, ST)                                                                                       \
+  with_k(k, [&](auto km) {                                                                                     \
+    hipLaunchKernelGGL((k_moe_combine<YT, ST, decltype(km)::value>), grid, kRT, 0, s, y, sym, scores, ssm, inv, T, \
+                       (int)k, A, N, out, som, nch);                                                           \
+  })
 #define CIN_COMB_S(YT)                          \
   if (s_dtype == CIN_DT_F32) CIN_COMB(YT, CIN_DT_F32);       \
   else if (s_dtype == CIN_DT_BF16) CIN_COMB(YT, CIN_DT_BF16); \
@@ -833,9 +807,11 @@ int cin_moe_combine_backward(const float* dout, int64_t sdm, const void* y, int 
     CIN_CHECK_ARG(k <= kMaxTopK, "moe_combine_backward: k must be at most %d", kMaxTopK);
     CIN_CHECK_ARG(cdiv(T * 64, kRT) < ((int64_t)1 << 31), "moe_combine_backward: grid too large");
     const unsigned grid = (unsigned)cdiv(T * 64, kRT);  // one wave per token
-#define CIN_TOK(YT, DT)                                                                          \
-  hipLaunchKernelGGL((k_moe_combine_bwd_tokens<YT, DT>), grid, kRT, 0, s, dout, sdm, y, sym, scores, \
-                     s_dtype, ssm, inv, T, (int)k, A, N, dy, sdym, dscores)
+#define CIN_TOK(YT, DT)                                                                                        \
+  with_k(k, [&](auto km) {                                                                                     \
+    hipLaunchKernelGGL((k_moe_combine_bwd_tokens<YT, DT, decltype(km)::value>), grid, kRT, 0, s, dout, sdm, y, sym, \
+                       scores, s_dtype, ssm, inv, T, (int)k, A, N, dy, sdym, dscores);                         \
+  })
 #define CIN_TOK_D(YT)                                        \
   if (dy_dtype == CIN_DT_F32) CIN_TOK(YT, CIN_DT_F32);       \
   else if (dy_dtype == CIN_DT_BF16) CIN_TOK(YT, CIN_DT_BF16); \

@@ -322,3 +322,39 @@ def test_routed_experts_tiny_gradients_against_an_fp32_chain(dev):
     for name, (e_fused, e_f16) in errs.items():
         assert e_fused <= 4e-2, name
         assert e_f16 >= 2.5 * e_fused, name
+
+
+# Every compiled bound on top-k (2, 4, 8, 16), under, at and over it; columns in one lane, a
+# partial and a whole step, several steps; dropped assignments
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("D,dtype", [(8, torch.float16), (520, torch.float32), (1100, torch.bfloat16),
+                                     (3080, torch.float16)])
+def test_combine_every_top_k(dev, k, D, dtype):
+    T, E = 61, 20
+    g = torch.Generator(device=dev).manual_seed(k * D)
+    idx = torch.rand(T, E + 2, generator=g, device=dev).argsort(dim=1)[:, :k] - 1  # ids -1 and E are dropped
+    perm, inv, _, _, _ = moe.moe_route(idx, E)
+    y = torch.randn(T * k, D, generator=g, device=dev).to(dtype)
+    sc = torch.rand(T, k, generator=g, device=dev)
+    dout = torch.randn(T, D, generator=g, device=dev)
+    pos = inv.view(T, k).long()
+    order = torch.where(pos < 0, torch.full_like(pos, T * k), pos).argsort(dim=1)
+    out, total = torch.zeros(T, D, device=dev), torch.zeros(T, D, device=dev)
+    dy = torch.zeros_like(y)
+    ds = torch.zeros(T, k, dtype=torch.float64, device=dev)
+    for j in range(k):  # a token's rows in sorted position order, product and sum rounded apart
+        slot = order[:, j:j + 1]
+        r, w = pos.gather(1, slot).squeeze(1), sc.gather(1, slot)
+        ok = (r >= 0).nonzero().squeeze(1)
+        rows = y[r[ok]].float()
+        out[ok] = out[ok] + rows * w[ok]
+        total[ok] = total[ok] + rows
+        dy[r[ok]] = (dout[ok] * w[ok]).to(dtype)
+        ds[ok, slot[ok, 0]] = (dout[ok].double() * rows.double()).sum(-1)
+    assert torch.equal(moe.moe_combine(y, sc, inv), out)
+    assert torch.equal(moe.moe_gather_sum(y, inv, k, torch.float32), total)
+    assert torch.equal(moe.moe_gather_sum(y, inv, k, dtype), total.to(dtype))
+    got_dy, got_ds = moe.moe_combine_backward(dout, y, sc, perm, inv)
+    assert torch.equal(got_dy, dy)
+    # D products summed in fp32 over at most D / 8 + 6 additions in a chain
+    assert ((got_ds.double() - ds).abs() <= (D / 8 + 8) * 2 ** -23 * D ** 0.5 * 16).all()
