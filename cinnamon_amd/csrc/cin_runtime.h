@@ -11,6 +11,9 @@ int cin_set_error(int code, const char* fmt, ...) __attribute__((format(printf, 
 // Check for a launch error after hipLaunchKernelGGL; returns CIN_OK or CIN_ERR_HIP.
 int cin_check_launch(const char* what);
 
+// Compute units of the current device.
+int cin_device_cus();
+
 #define CIN_CHECK_ARG(cond, ...)                    \
   do {                                              \
     if (!(cond)) return cin_set_error(CIN_ERR_ARG, __VA_ARGS__); \

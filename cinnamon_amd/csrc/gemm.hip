@@ -1738,8 +1738,6 @@ void with_tile(int64_t M, int64_t N, int64_t ncu, F launch) {
 
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
-// Compute units of the current device (the persistent grid runs one workgroup per CU),
-// looked up once per device.
 // The persistent kernels' epilogue for this C (pers::kEpi*); sce is the wgrad's expert
 // stride in elements (0 elsewhere).
 int pers_epi(int c_dtype, const void* C, int64_t ldc, int64_t sce) {
@@ -1748,18 +1746,6 @@ int pers_epi(int c_dtype, const void* C, int64_t ldc, int64_t sce) {
     return (a & 15) == 0 && ldc % 4 == 0 && sce % 4 == 0 ? pers::kEpiCounted32 : pers::kEpiDirect;
   if ((a & 15) == 0 && ldc % 8 == 0 && sce % 8 == 0) return pers::kEpiCounted16x4;
   return (a & 7) == 0 && ldc % 4 == 0 && sce % 4 == 0 ? pers::kEpiCounted16 : pers::kEpiDirect;
-}
-
-int device_cus() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cached[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    cached[dev] = n;
-  }
-  return cached[dev];
 }
 
 // The 256 x 256 kernels address a tile's operands by 32-bit offsets from its first row
@@ -1817,7 +1803,7 @@ int cin_gemm_fp8_bs(const uint8_t* A, int64_t lda, const float* sa, int64_t ssam
     hipLaunchKernelGGL(k_zero_rows16, grid, 256, 0, s, static_cast<uint16_t*>(C), M, N * es / 2, ldc * es / 2);
     return cin_check_launch("gemm_fp8_bs");
   }
-  const uint32_t ncu = (uint32_t)device_cus();
+  const uint32_t ncu = (uint32_t)cin_device_cus();
   const bool tile_fits = gt::offsets_fit(128, lda, ldb, K, ssam, ssak);
   if (K % big::TK == 0 && M >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak) &&
       !(tile_fits && rounds_sparse(cdiv(M, big::TM) * cdiv(N, big::TN), ncu))) {
@@ -1878,7 +1864,7 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
                     aligned16(A) && aligned16(B),
                 "grouped_gemm_fp8: A/B rows must be 16-byte aligned and K-contiguous");
   CIN_CHECK_ARG(ldc >= N, "grouped_gemm_fp8: bad C stride");
-  const int64_t ncu = device_cus();
+  const int64_t ncu = cin_device_cus();
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool big_ok = K % big::TK == 0 && T >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak);
   if (gt::offsets_fit(128, lda, ldb, K, ssam, ssak)) {
@@ -1981,7 +1967,7 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
                 "grouped_wgrad_fp8: operand rows too long for the 256 x 256 tile's 32-bit offsets");
   const int64_t tm = cdiv(N, big::TM), tn = cdiv(K, big::TN);
   CIN_CHECK_ARG(E * tm * tn < ((int64_t)1 << 31), "grouped_wgrad_fp8: grid too large");
-  const int64_t cus = device_cus();
+  const int64_t cus = cin_device_cus();
   // Up to four rounds of 256 x 256 tiles: ragged experts leave the persistent walk waiting for
   // the CUs that hold the longest tiles (and half-filled rounds), where the 128 x 128 tiles'
   // dispatch evens them out.  us, persistent / 128 x 128, Zipf(1.1) rows, T, E, N, K: 32768, 16,
@@ -2006,7 +1992,7 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
   if (E <= pers::kMaxWgradExperts) {
     // one workgroup per CU on the persistent walk; the counted epilogues need every expert's
     // dW aligned as the first one (sce a multiple of 4 elements)
-    const unsigned ncu = (unsigned)device_cus();
+    const unsigned ncu = (unsigned)cin_device_cus();
 #define CIN_LAUNCH_WGRAD_PERS(EPI_)                                                                   \
   hipLaunchKernelGGL(pers::k_grouped_wgrad_fp8_pers<EPI_>, ncu, big::kThreads, 0,                       \
                      static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, ldb, sb, ssbm, starts,   \

@@ -68,7 +68,7 @@ struct Tile {
   int nsub;
 };
 
-__device__ inline Tile tile_of(int64_t S, int64_t tiles_t, int64_t tiles_s, int xcd_rotate) {
+__device__ inline Tile tile_of(int64_t S, int64_t tiles_t, int64_t tiles_s, int xcd_rotate, int64_t kpw = kKPW) {
   int64_t tile = blockIdx.x;
   if (xcd_rotate) {
     const int64_t per = gridDim.x >> 3;
@@ -79,8 +79,8 @@ __device__ inline Tile tile_of(int64_t S, int64_t tiles_t, int64_t tiles_s, int 
   const int64_t rem = tile - t.b * tiles_t * tiles_s;
   t.tt = rem / tiles_s;
   t.sw = rem - t.tt * tiles_s;
-  t.s_begin = t.sw * kKPW;
-  t.s_end = t.s_begin + kKPW < S ? t.s_begin + kKPW : S;
+  t.s_begin = t.sw * kpw;
+  t.s_end = t.s_begin + kpw < S ? t.s_begin + kpw : S;
   t.nsub = (int)((t.s_end - t.s_begin + kKT - 1) / kKT);
   return t;
 }
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kMinWa
     const void* __restrict__ qin, const float* __restrict__ qs, const uint8_t* __restrict__ k8,
     const float* __restrict__ ks, const float* __restrict__ w, int64_t L, int64_t S, int64_t H,
     float softmax_scale, float* __restrict__ out, int64_t tiles_t, int64_t tiles_s, int xcd_rotate,
-    int vec, uint8_t* __restrict__ q8_out = nullptr, float* __restrict__ qs_out = nullptr) {
+    int vec, int64_t kpw, uint8_t* __restrict__ q8_out = nullptr, float* __restrict__ qs_out = nullptr) {
   constexpr int NC = (D + 127) / 128;           // 128-byte slices of d
   constexpr int RS = KeyStage<D>::RS;
   constexpr int OS = kKT + 4;                   // staging row stride (floats)
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kMinWa
   __shared__ __attribute__((aligned(16))) float ksl[2][kKT];
   __shared__ __attribute__((aligned(16))) float ost[4 * 16 * OS];
 
-  const Tile tl = tile_of(S, tiles_t, tiles_s, xcd_rotate);
+  const Tile tl = tile_of(S, tiles_t, tiles_s, xcd_rotate, kpw);
   const int64_t b = tl.b;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int l16 = lane & 15, kq = lane >> 4;
@@ -366,7 +366,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(kMinWa
             p[g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(kf[c], qf[g][c], p[g], 0, 0, 0, 0, 0, 0);
         }
         // (the results pass through one empty asm: all MFMAs issue before any of them is read)
-        if constexpr (HG == 4)
+        if constexpr (HG == 8)
+          asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(p[4]), "+v"(p[5]), "+v"(p[6]), "+v"(p[7]));
+        else if constexpr (HG == 4)
           asm volatile("" : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]));
         else if constexpr (HG == 2)
           asm volatile("" : "+v"(p[0]), "+v"(p[1]));
@@ -886,23 +888,39 @@ __global__ void k_indexer_wgrad_finish(const float* __restrict__ partial, const 
   dw[i] = (g * softmax_scale) * qs[i];
 }
 
+// Keys per workgroup of the 4-wave scoring kernels: kKPW, or a half or a quarter of it where
+// that many leave CUs without a workgroup.  B, L, S, H, d: 2, 777, 4100, 8, 64: 512 keys (234
+// workgroups) 28.0 us, 256 keys (442) 24.4, 128 keys (858) 30.8; 1, 512, 4096, 16, 64: 56.3, 128
+// keys 21.6; 2, 300, 3000, 2, 192: 23.7, 15.4.
+int64_t keys_per_workgroup(int64_t token_tiles, int64_t S) {
+  int64_t kpw = kKPW;
+  while (kpw > kKT && token_tiles * cdiv(S, kpw) < cin_device_cus()) kpw /= 2;
+  return kpw;
+}
+
+// Whether the 8-wave kernels (64 tokens x 1024 keys) have a workgroup for at least half of the
+// CUs; with fewer, the 4-wave kernels and shorter key ranges finish first.
+bool pair_fills(int64_t B, int64_t tiles_t, int64_t S) {
+  return 2 * B * tiles_t * cdiv(S, kKPW2) >= cin_device_cus();
+}
+
 template <int D, int HG>
 void launch_indexer(unsigned grid, hipStream_t st, const uint8_t* q8, const float* qs,
                     const uint8_t* k8, const float* ks, const float* w, int64_t L, int64_t S,
                     int64_t H, float softmax_scale, float* out, int64_t tiles_t, int64_t tiles_s,
-                    int xcd_rotate, int vec) {
+                    int xcd_rotate, int vec, int64_t kpw) {
   hipLaunchKernelGGL((k_indexer_scores_fp8<D, HG>), grid, kThreads, 0, st, q8, qs, k8, ks, w, L, S,
-                     H, softmax_scale, out, tiles_t, tiles_s, xcd_rotate, vec);
+                     H, softmax_scale, out, tiles_t, tiles_s, xcd_rotate, vec, kpw);
 }
 
 template <int D, int HG>
 void launch_indexer_q(int q_dtype, unsigned grid, hipStream_t st, const void* q, const uint8_t* k8,
                       const float* ks, const float* w, int64_t L, int64_t S, int64_t H,
                       float softmax_scale, float* out, int64_t tiles_t, int64_t tiles_s,
-                      int xcd_rotate, int vec, uint8_t* q8_out, float* qs_out) {
+                      int xcd_rotate, int vec, int64_t kpw, uint8_t* q8_out, float* qs_out) {
 #define CIN_IQ_LAUNCH(DT)                                                                         \
   hipLaunchKernelGGL((k_indexer_scores_fp8<D, HG, DT>), grid, kThreads, 0, st, q, nullptr, k8, ks, w, \
-                     L, S, H, softmax_scale, out, tiles_t, tiles_s, xcd_rotate, vec, q8_out, qs_out)
+                     L, S, H, softmax_scale, out, tiles_t, tiles_s, xcd_rotate, vec, kpw, q8_out, qs_out)
   if (q_dtype == CIN_DT_BF16)
     CIN_IQ_LAUNCH(CIN_DT_BF16);
   else if (q_dtype == CIN_DT_F16)
@@ -953,13 +971,13 @@ int cin_indexer_scores_fp8(const uint8_t* q8, const float* q_scale, const uint8_
   CIN_CHECK_ARG(q8 && q_scale && k8 && k_scale && weights && scores, "indexer_scores_fp8: null pointer");
   CIN_CHECK_ARG((((uintptr_t)q8) & 15) == 0 && (((uintptr_t)k8) & 15) == 0,
                 "indexer_scores_fp8: code buffers must be 16-byte aligned");
-  const int64_t tiles_t = cdiv(L, kTT), tiles_s = cdiv(S, kKPW);
+  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S), tiles_s = cdiv(S, kpw);
   CIN_CHECK_ARG(B * tiles_t * tiles_s < ((int64_t)1 << 31), "indexer_scores_fp8: grid too large");
   const unsigned grid = (unsigned)(B * tiles_t * tiles_s);
   const int xcd_rotate = grid % 8 == 0;
   const int vec = S % 4 == 0 && (((uintptr_t)k_scale) & 15) == 0 && (((uintptr_t)scores) & 15) == 0;
   const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (d <= 128 && H <= 4 && S > kKPW) {
+  if (d <= 128 && H <= 4 && S > kKPW && pair_fills(B, tiles_t, S)) {
     // 8 waves per 64 tokens x 1024 keys: q's codes read once per 1024 keys
     const int64_t tiles_s2 = cdiv(S, kKPW2);
     const unsigned grid2 = (unsigned)(B * tiles_t * tiles_s2);
@@ -976,12 +994,21 @@ int cin_indexer_scores_fp8(const uint8_t* q8, const float* q_scale, const uint8_
     }
     return cin_check_launch("indexer_scores_fp8");
   }
-  switch (d / 32) {
 #define CIN_INDEXER_CASE(n, hg)                                                                 \
   case n:                                                                                       \
     launch_indexer<32 * n, hg>(grid, st, q8, q_scale, k8, k_scale, weights, L, S, H,            \
-                               softmax_scale, scores, tiles_t, tiles_s, xcd_rotate, vec);       \
+                               softmax_scale, scores, tiles_t, tiles_s, xcd_rotate, vec, kpw);  \
     break;
+  if (d <= 128 && H > 4) {
+    // eight heads' fragments at once: with four, every 128-key sub-tile loaded each group's q
+    // again (16 x 1024 tokens, 8 heads, d 128: 63.7 -> 46.7 us with the quantization; 1 x 2048
+    // tokens, 8 heads, d 128: 38.7 -> 19.0 with shorter key ranges too)
+    switch (d / 32) {
+      CIN_INDEXER_CASE(1, 8) CIN_INDEXER_CASE(2, 8) CIN_INDEXER_CASE(3, 8) CIN_INDEXER_CASE(4, 8)
+    }
+    return cin_check_launch("indexer_scores_fp8");
+  }
+  switch (d / 32) {
     CIN_INDEXER_CASE(1, 4) CIN_INDEXER_CASE(2, 4) CIN_INDEXER_CASE(3, 4) CIN_INDEXER_CASE(4, 4)
     CIN_INDEXER_CASE(5, 2) CIN_INDEXER_CASE(6, 2) CIN_INDEXER_CASE(7, 2) CIN_INDEXER_CASE(8, 2)
 #undef CIN_INDEXER_CASE
@@ -1018,7 +1045,7 @@ int cin_indexer_scores_fp8_q(const void* q, int q_dtype, const uint8_t* k8, cons
   CIN_CHECK_ARG((((uintptr_t)k8) & 15) == 0, "indexer_scores_fp8_q: k8 must be 16-byte aligned");
   const hipStream_t st = static_cast<hipStream_t>(stream);
   const int vec = S % 4 == 0 && (((uintptr_t)k_scale) & 15) == 0 && (((uintptr_t)scores) & 15) == 0;
-  if (d <= 128 && S > kKPW) {
+  if (d <= 128 && S > kKPW && pair_fills(B, cdiv(L, kTT), S)) {
     // 8 waves per 64 tokens x 1024 keys: q read and quantized once per 1024 keys
     const int64_t tiles_t2 = cdiv(L, kTT), tiles_s2 = cdiv(S, kKPW2);
     CIN_CHECK_ARG(B * tiles_t2 * tiles_s2 < ((int64_t)1 << 31), "indexer_scores_fp8_q: grid too large");
@@ -1035,7 +1062,7 @@ int cin_indexer_scores_fp8_q(const void* q, int q_dtype, const uint8_t* k8, cons
     }
     return cin_check_launch("indexer_scores_fp8_q");
   }
-  const int64_t tiles_t = cdiv(L, kTT), tiles_s = cdiv(S, kKPW);
+  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S), tiles_s = cdiv(S, kpw);
   CIN_CHECK_ARG(B * tiles_t * tiles_s < ((int64_t)1 << 31), "indexer_scores_fp8_q: grid too large");
   const unsigned grid = (unsigned)(B * tiles_t * tiles_s);
   const int xcd_rotate = grid % 8 == 0;
@@ -1043,7 +1070,7 @@ int cin_indexer_scores_fp8_q(const void* q, int q_dtype, const uint8_t* k8, cons
 #define CIN_INDEXER_Q_CASE(n, hgv)                                                                  \
   case n:                                                                                           \
     launch_indexer_q<32 * n, hgv>(q_dtype, grid, st, q, k8, k_scale, weights, L, S, H, softmax_scale, \
-                                  scores, tiles_t, tiles_s, xcd_rotate, vec, q8, q_scale);          \
+                                  scores, tiles_t, tiles_s, xcd_rotate, vec, kpw, q8, q_scale);     \
     break;
     CIN_INDEXER_Q_CASE(1, 4) CIN_INDEXER_Q_CASE(2, 4) CIN_INDEXER_Q_CASE(3, 4) CIN_INDEXER_Q_CASE(4, 4)
     CIN_INDEXER_Q_CASE(5, 2) CIN_INDEXER_Q_CASE(6, 2) CIN_INDEXER_Q_CASE(7, 2) CIN_INDEXER_Q_CASE(8, 2)

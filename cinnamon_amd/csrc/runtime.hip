@@ -22,6 +22,19 @@ int cin_check_launch(const char* what) {
   return CIN_OK;
 }
 
+// (looked up once per device; two threads that look it up together store the same value)
+int cin_device_cus() {
+  static int cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cached[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    cached[dev] = n;
+  }
+  return cached[dev];
+}
+
 extern "C" {
 
 int cin_abi_version(void) { return 3; }

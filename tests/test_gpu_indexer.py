@@ -201,3 +201,26 @@ def test_rejects_unsupported_head_dims(dev):
     w = torch.randn(1, 8, 2, device=dev)
     with pytest.raises(AssertionError):
         kernels.indexer_scores_fp8(q, k, w, 0.1)
+
+
+# The 8-wave form's edges in a grid large enough for it (with fewer than one workgroup for two
+# CUs the 4-wave kernels run): a second half with 1 key, an empty second half in the last
+# range, three ranges, one head
+@pytest.mark.parametrize("B,L,S,H,d,dtype", [
+    (64, 100, 600, 4, 128, torch.bfloat16),
+    (32, 65, 1500, 4, 64, torch.float16),
+    (22, 77, 2049, 2, 32, torch.bfloat16),
+    (128, 64, 1088, 1, 128, torch.float32),
+])
+def test_fused_q_quantization_equals_the_two_calls_full_grid(dev, B, L, S, H, d, dtype):
+    test_fused_q_quantization_equals_the_two_calls(dev, B, L, S, H, d, dtype)
+
+
+# Eight heads at once: a partial, a whole, two and more groups; key ranges of 512, 256 and 128
+@pytest.mark.parametrize("B,L,S,H,d,dtype", [
+    (1, 70, 1100, 5, 128, torch.bfloat16), (2, 64, 300, 8, 32, torch.float32), (1, 33, 700, 9, 96, torch.float16),
+    (1, 20, 1500, 16, 64, torch.bfloat16), (9, 300, 900, 8, 64, torch.bfloat16), (20, 500, 520, 6, 32, torch.bfloat16),
+    (3, 129, 513, 3, 160, torch.bfloat16),
+])
+def test_scores_of_many_heads(dev, B, L, S, H, d, dtype):
+    test_scores_match_the_oracle(dev, B, L, S, H, d, dtype)
