@@ -1759,12 +1759,14 @@ bool big_offsets_fit(int64_t lda, int64_t ldb, int64_t klen, int64_t ssam, int64
 }
 
 // Whether a grid of 256 x 256 tiles leaves so many CUs idle in its last round that the 128 x
-// 128 and smaller tiles finish first: at most 5/8 of the rounds' CU slots used.  us, 256 x 256 /
-// smaller tiles: 64 of 256 CUs (4096, 1024, 1024) 14.9 / 11.5 and (2048, 2048, 2048) 24.5 / 16.0;
-// 128 (4096, 2048, 4096) 44.5 / 40.9; 264 (8448, 2048, 2048) 55.8 / 50.4; 320 (10000, 2048, 1024)
-// 33.6 / 31.8; and the other way round: 192 (6144, 2048, 4096) 48.8 / 59.4, 384 (12288, 2048,
-// 2048) 55.0 / 61.4.
-bool rounds_sparse(int64_t tiles, int64_t ncu) { return tiles * 8 <= cdiv(tiles, ncu) * ncu * 5; }
+// 128 and smaller tiles finish first: up to half a round (whose 128 x 128 tiles, two a CU, are
+// one round), or an eighth past a full one.  us, 256 x 256 / smaller tiles, by tiles on 256 CUs:
+// 64 (4096, 1024, 1024) 14.9 / 11.5 and (2048, 2048, 2048) 24.5 / 16.0; 128 (4096, 2048, 4096) 44.5 /
+// 40.9; 136 (4352, 2048, 4096) 44.4 / 57.5; 160 (2560, 4096, 1024) 17.2 / 22.6; 264 (8448, 2048, 4096)
+// 96.6 / 90.2; 288 (9216, 2048, 4096) 96.0 / 93.3; 320 (10240, 2048, 4096) 94.6 / 99.2.
+bool rounds_sparse(int64_t tiles, int64_t ncu) {
+  return tiles * 2 <= ncu || (tiles > ncu && tiles * 8 <= ncu * 9);
+}
 
 }  // namespace
 
