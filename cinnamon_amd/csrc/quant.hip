@@ -1599,23 +1599,37 @@ __global__ __launch_bounds__(kThreads) void k_dequant(const uint8_t* __restrict_
 }
 
 // ---------------------------------------------------------------------------
-// Byte transpose through a 64x64 LDS tile.
+// Byte transpose, 128 x 128 tiles: a thread takes 8 bytes of each of 8 rows (rows may start
+// anywhere: the loads are unaligned ones), transposes them in registers, and the tile leaves
+// LDS as 16-byte pieces of the output rows where those are aligned.  Bound by latency at these
+// sizes (one tile a workgroup): 4000 x 1500 bytes 10.3 -> 8.0 us, 7168 x 2048 17.8 -> 7.8, against
+// one byte a thread and step through 64 x 64 tiles.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kThreads) void k_transpose_u8(const uint8_t* __restrict__ src,
                                                            int64_t R, int64_t C, int64_t lds,
                                                            uint8_t* __restrict__ dst,
                                                            int64_t ldd) {
-  __shared__ uint8_t tile[64][65];
-  const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
-  for (int i = threadIdx.x; i < 64 * 64; i += kThreads) {
-    const int rr = i >> 6, cc = i & 63;
-    if (r0 + rr < R && c0 + cc < C) tile[rr][cc] = src[(r0 + rr) * lds + c0 + cc];
+  __shared__ TileT tile;
+  const int lane16 = threadIdx.x & 15, rg = threadIdx.x >> 4;
+  const int64_t r0 = (int64_t)blockIdx.y * 128, c0 = (int64_t)blockIdx.x * 128;
+  const int64_t r = r0 + rg * 8, c = c0 + lane16 * 8;
+  uint32_t rows[8][2], cols[8][2];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) rows[i][0] = rows[i][1] = 0u;
+  if (c + 8 <= C) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (r + i < R) __builtin_memcpy(rows[i], src + (r + i) * lds + c, 8);
+  } else if (c < C) {
+    for (int i = 0; i < 8; ++i)
+      for (int j = 0; j < 8; ++j)
+        if (r + i < R && c + j < C) rows[i][j >> 2] |= (uint32_t)src[(r + i) * lds + c + j] << (8 * (j & 3));
   }
+  t8x8(rows, cols);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) put_col8(tile, lane16 * 8 + j, rg, cols[j][0], cols[j][1]);
   __syncthreads();
-  for (int i = threadIdx.x; i < 64 * 64; i += kThreads) {
-    const int cc = i >> 6, rr = i & 63;
-    if (r0 + rr < R && c0 + cc < C) dst[(c0 + cc) * ldd + r0 + rr] = tile[rr][cc];
-  }
+  store_tile_t(tile, dst, ldd, c0, C, r0, (int)(R - r0 < 128 ? R - r0 : 128));
 }
 
 
@@ -2532,7 +2546,7 @@ int cin_transpose_u8(const uint8_t* src, int64_t R, int64_t C, int64_t lds, uint
   CIN_CHECK_ARG(src && dst && lds >= C && ldd >= R, "transpose_u8: bad pointer or stride");
   CIN_CHECK_ARG(cdiv(R, 64) < 65536, "transpose_u8: too many rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
-  dim3 grid((unsigned)cdiv(C, 64), (unsigned)cdiv(R, 64));
+  dim3 grid((unsigned)cdiv(C, 128), (unsigned)cdiv(R, 128));
   hipLaunchKernelGGL(k_transpose_u8, grid, kThreads, 0, s, src, R, C, lds, dst, ldd);
   return cin_check_launch("transpose_u8");
 }

@@ -412,3 +412,12 @@ def test_backward_padded_equals_unpadded(kern, dev, M, N, K, dtype):
             assert torch.count_nonzero(a[:, M:]) == 0
             a = a[:, :M]
         assert torch.equal(a, b)
+
+
+# whole, partial and single-byte tiles; rows that start on any byte
+@pytest.mark.parametrize("R,C,off", [(1, 1, 0), (7, 130, 0), (128, 128, 0), (129, 1500, 3), (4000, 1500, 0),
+                                     (64, 4097, 1), (272, 136, 8)])
+def test_transpose_bytes(kern, dev, R, C, off):
+    g = torch.Generator().manual_seed(R + C)
+    src = torch.randint(0, 256, (R, C + off), generator=g, dtype=torch.uint8).to(dev)[:, off:]
+    assert torch.equal(kern._transpose_u8_op(src), src.t().contiguous())
