@@ -6,8 +6,7 @@
 // Operands are rounded to fp16 (round-to-nearest-even) as the reference's
 // a.to(tl.float16) / b.to(tl.float16) do, the products are summed in fp32 by
 // v_mfma_f32_16x16x32_f16, and the result is stored as fp16 (RNE).  One launch covers all
-// experts: a workgroup finds its (expert, 128-row tile) by scanning the device-side
-// ranges, so there is no host synchronisation and no grid sized by the largest expert.
+// experts: a workgroup finds its (expert, row tile) from the device-side ranges, so there is no host synchronisation and no grid sized by the largest expert.
 // Rows outside every expert range are not written (the reference returns torch.empty).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -20,8 +19,7 @@ using namespace cin;
 
 namespace {
 
-constexpr int BM = 128, BN = 128, BK = 64;  // workgroup tile, K step per LDS stage
-constexpr int kThreads = 256;               // 4 waves in 2 x 2, wave tile 64 x 64
+constexpr int BK = 64;                      // K step per LDS stage
 constexpr int kRowBytes = BK * 2;           // one fp16 tile row: 8 chunks of 16 bytes
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
@@ -31,176 +29,16 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // 128-byte rows: conflict-free fragment reads)
 __device__ inline int swz_f(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-template <int DT>
-__device__ inline float elem(const void* p, int64_t i) {
-  if constexpr (DT == CIN_DT_BF16) return __uint_as_float(((uint32_t)((const uint16_t*)p)[i]) << 16);
-  else if constexpr (DT == CIN_DT_F16) return (float)((const _Float16*)p)[i];
-  else return ((const float*)p)[i];
-}
-
-// 32 consecutive elements of one row (zero past `nvalid`), rounded to fp16, as 4 chunks.
-// VEC: the 32 elements are in range and 16-byte aligned (vector loads).
-template <int DT, bool VEC>
-__device__ inline void load32(const void* base, int64_t off, int64_t nvalid, h8 (&o)[4]) {
-  if constexpr (VEC) {
-    if constexpr (DT == CIN_DT_F32) {
-      const float4* p = reinterpret_cast<const float4*>(static_cast<const float*>(base) + off);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float4 a = p[2 * c], b = p[2 * c + 1];
-        o[c] = h8{(_Float16)a.x, (_Float16)a.y, (_Float16)a.z, (_Float16)a.w,
-                  (_Float16)b.x, (_Float16)b.y, (_Float16)b.z, (_Float16)b.w};
-      }
-    } else if constexpr (DT == CIN_DT_F16) {
-      const h8* p = reinterpret_cast<const h8*>(static_cast<const _Float16*>(base) + off);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) o[c] = p[c];
-    } else {
-      const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(base) + off);
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint4 w = p[c];
-        const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          o[c][2 * e] = (_Float16)bf16_lo(ws[e]);
-          o[c][2 * e + 1] = (_Float16)bf16_hi(ws[e]);
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int k = c * 8 + e;
-        o[c][e] = k < nvalid ? (_Float16)elem<DT>(base, off + k) : (_Float16)0.0f;
-      }
-  }
-}
-
-template <int ADT, int BDT, bool VEC>
-__global__ __launch_bounds__(kThreads) void k_grouped_gemm_f16(
-    const void* __restrict__ A, int64_t lda, const void* __restrict__ B, int64_t sbe, int64_t ldb,
-    const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t T,
-    int64_t N, int64_t K, _Float16* __restrict__ C, int64_t ldc, uint32_t tiles_n) {
-  __shared__ __attribute__((aligned(16))) uint8_t sa[2][BM * kRowBytes];
-  __shared__ __attribute__((aligned(16))) uint8_t sb[2][BN * kRowBytes];
-  const uint32_t tile = blockIdx.x / tiles_n, tn = blockIdx.x - tile * tiles_n;
-  // (expert, 128-row tile) of this workgroup
-  int64_t seen = 0, e = -1, r0 = 0, r1 = 0;
-  for (int64_t x = 0; x < E; ++x) {
-    int64_t s0, s1;
-    clamp_range(starts, ends, x, T, s0, s1);
-    const int64_t nt = (s1 - s0 + BM - 1) / BM;
-    if ((int64_t)tile < seen + nt) {
-      e = x;
-      r0 = s0 + ((int64_t)tile - seen) * BM;
-      r1 = s1;
-      break;
-    }
-    seen += nt;
-  }
-  if (e < 0) return;  // surplus workgroup, before any barrier
-  const int nr = (int)(r1 - r0 < BM ? r1 - r0 : BM);
-  const int64_t n0 = (int64_t)tn * BN;
-  const uint8_t* Be = static_cast<const uint8_t*>(B) + e * sbe * (BDT == CIN_DT_F32 ? 4 : 2);
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int l16 = lane & 15, kq = lane >> 4;
-  // loads: thread = (tile row tid / 2, 32-element half tid % 2)
-  const int lr = tid >> 1, lh = tid & 1;
-  const bool arow = lr < nr, brow = n0 + lr < N;
-  const int64_t aoff = (r0 + lr) * lda, boff = (n0 + lr) * ldb;
-
-  v4f acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-
-  h8 ga[4], gb[4];
-  auto fetch = [&](int64_t k0) {
-    const int64_t k = k0 + lh * 32;
-    const int64_t nv = K - k;
-    if (arow) load32<ADT, VEC>(A, aoff + k, nv, ga);
-    else for (int c = 0; c < 4; ++c) ga[c] = h8{};
-    if (brow) load32<BDT, VEC>(Be, boff + k, nv, gb);
-    else for (int c = 0; c < 4; ++c) gb[c] = h8{};
-  };
-  auto store = [&](int st) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int slot = (lh * 4 + c) ^ swz_f(lr);
-      *reinterpret_cast<h8*>(&sa[st][lr * kRowBytes + slot * 16]) = ga[c];
-      *reinterpret_cast<h8*>(&sb[st][lr * kRowBytes + slot * 16]) = gb[c];
-    }
-  };
-  // fragment: row `row`, K elements [8 q, 8 q + 8) of k-step ks (chunk 4 ks + q)
-  auto frag = [&](const uint8_t* base, int row, int ks) -> h8 {
-    const int slot = (4 * ks + kq) ^ swz_f(row);
-    return *reinterpret_cast<const h8*>(base + row * kRowBytes + slot * 16);
-  };
-
-  const int nkt = (int)((K + BK - 1) / BK);
-  fetch(0);
-  store(0);
-  __syncthreads();
-  for (int kt = 0; kt < nkt; ++kt) {
-    const int st = kt & 1;
-    if (kt + 1 < nkt) fetch((int64_t)(kt + 1) * BK);
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      h8 bfr[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) bfr[j] = frag(sb[st], wn * 64 + j * 16 + l16, ks);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const h8 afr = frag(sa[st], wm * 64 + i * 16 + l16, ks);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bfr[j], afr, acc[i][j], 0, 0, 0);
-      }
-    }
-    if (kt + 1 < nkt) store(st ^ 1);
-    __syncthreads();
-  }
-
-  // epilogue: lane holds C[m][n .. n+3]
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int m = wm * 64 + i * 16 + l16;
-    if (m >= nr) continue;
-    _Float16* crow = C + (r0 + m) * ldc;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int64_t n = n0 + wn * 64 + j * 16 + kq * 4;
-      const _Float16 h0 = (_Float16)acc[i][j][0], h1 = (_Float16)acc[i][j][1];
-      const _Float16 h2 = (_Float16)acc[i][j][2], h3 = (_Float16)acc[i][j][3];
-      if (n + 4 <= N && (((uintptr_t)(crow + n)) & 7) == 0) {
-        typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-        *reinterpret_cast<h4*>(crow + n) = h4{h0, h1, h2, h3};
-      } else {
-        const _Float16 hv[4] = {h0, h1, h2, h3};
-        for (int r = 0; r < 4; ++r)
-          if (n + r < N) crow[n + r] = hv[r];
-      }
-    }
-  }
-}
-
 // ---------------------------------------------------------------------------
-// The same product for operands whose rows are 16-byte aligned (K % 8 == 0): workgroup tiles
-// of 16 MT WM x 16 NT WN, K steps of 64 through two LDS stages.  Each thread keeps the next
-// step's operands in flight in registers, in their own dtype, while the current step's MFMAs
-// run, then converts them to fp16 on the way into LDS: no converted copy of the weights is
-// ever stored.  A wider tile reads fp32 weights less often: with 256 x 256 tiles a step's 96 KB
-// of operands (fp32 weights, 16-bit rows) take about 1500 cycles at 64 B / clk and its MFMAs
-// 2048, with 128 x 128 tiles 768 and 512.  Rows past an expert or past N and elements past K
-// come from out-of-range lanes, which read as zero.  32768 Zipf rows, 16 experts, 2048 x 1024,
-// bf16 rows: 217 us with fp32 weights, 174 with bf16 (k_grouped_gemm_f16 400 and 280, the same
-// bits): 0.63 and 0.79 PFLOP/s, with 1088 tiles in five rounds of 256.
+// Workgroup tiles of 16 MT WM x 16 NT WN, K steps of 64 through two LDS stages.  Each thread
+// keeps the next step's operands in flight in registers, in their own dtype, while the current
+// step's MFMAs run, then converts them to fp16 on the way into LDS: no converted copy of the
+// weights is ever stored.  A wider tile reads fp32 weights less often: with 256 x 256 tiles a
+// step's 96 KB of operands (fp32 weights, 16-bit rows) take about 1500 cycles at 64 B / clk and
+// its MFMAs 2048, with 128 x 128 tiles 768 and 512.  Rows past an expert or past N and elements
+// past K read as zero.  32768 Zipf rows, 16 experts, 2048 x 1024, bf16 rows: 217 us with fp32
+// weights, 174 with bf16 (128 x 128 tiles that waited for each step's loads: 400 and 280, the
+// same bits): 0.63 and 0.79 PFLOP/s, with 1088 tiles in five rounds of 256.
 // ---------------------------------------------------------------------------
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -212,9 +50,13 @@ __device__ inline h2 to_h2(float a, float b) { return __builtin_convertvector(f2
 
 // One operand's share of a K step: ROWS rows x 64 elements over THREADS threads, 16 bytes of
 // the source dtype per thread and operation.
-template <int DT, int ROWS, int THREADS>
+// ALIGNED: rows start on 16 bytes, K % 8 == 0 and a tile's rows lie within 2^31 bytes (buffer
+// loads, out-of-range lanes read zero).  Otherwise the 16 bytes come from 64-bit addresses and
+// any element alignment, and the last ones of a row element by element.
+template <int DT, int ROWS, int THREADS, bool ALIGNED>
 struct Operand {
   static constexpr int kEs = DT == CIN_DT_F32 ? 4 : 2;
+  static constexpr int kPer = 16 / kEs;
   static constexpr int kLanes = 64 * kEs / 16;  // threads of one row
   static constexpr int kOps = ROWS * kLanes / THREADS;
   static constexpr int kRowsPerOp = THREADS / kLanes;
@@ -222,23 +64,58 @@ struct Operand {
   v4u r[kOps];
   __amdgpu_buffer_rsrc_t rsrc;
   uint32_t off, step;
+  const uint8_t* p;  // !ALIGNED: the thread's first element of operation 0
+  int64_t stride;    // bytes between operations
+  int row, rows;
   uint32_t lds;  // byte offset of operation 0 in a stage
   int k;         // first element of the thread's 16 bytes within a step
 
-  __device__ __forceinline__ void init(const void* p, int64_t ld, int rows, int64_t K, int tid) {
-    rsrc = make_rsrc(p, ((int64_t)(rows - 1) * ld + K) * kEs);
-    const int row = tid / kLanes, c = tid % kLanes;
-    k = c * (16 / kEs);
-    off = (uint32_t)(row * ld * kEs) + c * 16;
-    step = (uint32_t)(kRowsPerOp * ld * kEs);
+  __device__ __forceinline__ void init(const void* base, int64_t ld, int rows_, int64_t K, int tid) {
+    row = tid / kLanes;
+    rows = rows_;
+    const int c = tid % kLanes;
+    k = c * kPer;
+    if constexpr (ALIGNED) {
+      rsrc = make_rsrc(base, ((int64_t)(rows - 1) * ld + K) * kEs);
+      off = (uint32_t)(row * ld * kEs) + c * 16;
+      step = (uint32_t)(kRowsPerOp * ld * kEs);
+    } else {
+      p = static_cast<const uint8_t*>(base) + (row * ld + k) * kEs;
+      stride = kRowsPerOp * ld * kEs;
+    }
     const int chunk = DT == CIN_DT_F32 ? c >> 1 : c;
     lds = (uint32_t)(row * kRowBytes + ((chunk ^ swz_f(row)) << 4) + (DT == CIN_DT_F32 ? (c & 1) * 8 : 0));
   }
   __device__ __forceinline__ void fetch(int64_t k0, int64_t K) {
-    const uint32_t out = k0 + k < K ? 0u : kOut;
+    if constexpr (ALIGNED) {
+      const uint32_t out = k0 + k < K ? 0u : kOut;
 #pragma unroll
-    for (int i = 0; i < kOps; ++i)
-      r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (off + i * step) | out, (uint32_t)(k0 * kEs), 0);
+      for (int i = 0; i < kOps; ++i)
+        r[i] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, (off + i * step) | out, (uint32_t)(k0 * kEs), 0);
+    } else {
+      const int64_t left = K - k0 - k;  // elements of the row from the thread's first one on
+      if (left >= kPer) {
+#pragma unroll
+        for (int i = 0; i < kOps; ++i) {
+          r[i] = v4u{0u, 0u, 0u, 0u};
+          if (row + i * kRowsPerOp < rows) __builtin_memcpy(&r[i], p + i * stride + k0 * kEs, 16);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < kOps; ++i) {
+          r[i] = v4u{0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int e = 0; e < kPer; ++e) {
+            if (e >= left || row + i * kRowsPerOp >= rows) continue;
+            const uint8_t* q = p + i * stride + (k0 + e) * kEs;
+            if constexpr (kEs == 4)
+              r[i][e] = *reinterpret_cast<const uint32_t*>(q);
+            else
+              r[i][e >> 1] |= (uint32_t)*reinterpret_cast<const uint16_t*>(q) << (16 * (e & 1));
+          }
+        }
+      }
+    }
   }
   __device__ __forceinline__ void store(uint8_t* stage) const {
 #pragma unroll
@@ -276,7 +153,7 @@ using W256 = Cfg16<2, 4, 8, 4>;    // 8 waves of 128 x 64
 using W128 = Cfg16<4, 2, 2, 4>;    // 8 waves of 32 x 64, two workgroups a CU
 using W64x128 = Cfg16<2, 2, 2, 4>; // 4 waves of 32 x 64, three workgroups a CU
 
-template <class C, int ADT, int BDT>
+template <class C, int ADT, int BDT, bool ALIGNED>
 __global__ __launch_bounds__(C::kThreads, 2) void k_grouped_gemm_f16_tile(
     const void* __restrict__ A, int64_t lda, const void* __restrict__ B, int64_t sbe, int64_t ldb,
     const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t T,
@@ -300,8 +177,8 @@ __global__ __launch_bounds__(C::kThreads, 2) void k_grouped_gemm_f16_tile(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / C::WN, wn = wave % C::WN;
   const int l16 = lane & 15, kq = lane >> 4;
-  Operand<ADT, C::TM, C::kThreads> oa;
-  Operand<BDT, C::TN, C::kThreads> ob;
+  Operand<ADT, C::TM, C::kThreads, ALIGNED> oa;
+  Operand<BDT, C::TN, C::kThreads, ALIGNED> ob;
   oa.init(static_cast<const uint8_t*>(A) + r0 * lda * oa.kEs, lda, nr, K, tid);
   ob.init(static_cast<const uint8_t*>(B) + (e * sbe + n0 * ldb) * ob.kEs, ldb, nc, K, tid);
   const int fsw = swz_f(l16);
@@ -391,11 +268,12 @@ struct Args {
   int64_t ldc;
 };
 
-template <class C, int ADT, int BDT>
+template <class C, int ADT, int BDT, bool ALIGNED>
 void launch_tile(const Args& a, hipStream_t s) {
   const int64_t tm = cdiv(a.T, C::TM) + a.E - 1, tn = cdiv(a.N, C::TN);
-  hipLaunchKernelGGL((k_grouped_gemm_f16_tile<C, ADT, BDT>), (unsigned)(tm * tn), C::kThreads, 0, s, a.A, a.lda, a.B,
-                     a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C, a.ldc, (uint32_t)tm, (uint32_t)tn);
+  hipLaunchKernelGGL((k_grouped_gemm_f16_tile<C, ADT, BDT, ALIGNED>), (unsigned)(tm * tn), C::kThreads, 0, s, a.A,
+                     a.lda, a.B, a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C, a.ldc, (uint32_t)tm,
+                     (uint32_t)tn);
 }
 
 template <int ADT, int BDT>
@@ -404,25 +282,24 @@ void launch(const Args& a, hipStream_t s) {
   const bool rows16 = ((uintptr_t)a.A % 16) == 0 && ((uintptr_t)a.B % 16) == 0 && (a.lda * ea) % 16 == 0 &&
                       (a.ldb * eb) % 16 == 0 && (a.sbe * eb) % 16 == 0;
   const int64_t lim = (int64_t)1 << 31;  // lane offsets from a tile's first row
-  if (rows16 && a.K > 0 && a.K % 8 == 0 && (256 * a.lda + a.K) * ea < lim && (256 * a.ldb + a.K) * eb < lim) {
+  const bool few = a.T <= 64 * a.E && (cdiv(a.T, 64) + a.E) * cdiv(a.N, 128) < lim;
+  if (rows16 && a.K % 8 == 0 && (256 * a.lda + a.K) * ea < lim && (256 * a.ldb + a.K) * eb < lim) {
     // us, 256 x 256 / 128 x 128 / 64 x 128 tiles, fp32 and bf16 weights, T, E, N, K: 32768, 16, 2048,
     // 1024 (four rounds of 256 x 256): 217, 174 / 236, 208 / 297, 240; 16384 (two): 120, 109 / 120,
     // 105 / 151, 123; 8192 (one): 76, 67 / 69, 60 / 86, 69; 1024 (64 rows an expert): 37, 34 / 31, 24 /
     // 33, 19; 64: 37, 34 / 22, 17 / 22, 15.
     if (a.T / 256 * cdiv(a.N, 256) >= 512)
-      launch_tile<W256, ADT, BDT>(a, s);
-    else if (a.T <= 64 * a.E && (cdiv(a.T, 64) + a.E) * cdiv(a.N, 128) < lim)
-      launch_tile<W64x128, ADT, BDT>(a, s);
+      launch_tile<W256, ADT, BDT, true>(a, s);
+    else if (few)
+      launch_tile<W64x128, ADT, BDT, true>(a, s);
     else
-      launch_tile<W128, ADT, BDT>(a, s);
-    return;
+      launch_tile<W128, ADT, BDT, true>(a, s);
+  } else if (few) {
+    // (31899, 16, 256, 1315, bf16: 842 us element by element, 65 so; 696, 32, 368, 541: 149, 16)
+    launch_tile<W64x128, ADT, BDT, false>(a, s);
+  } else {
+    launch_tile<W128, ADT, BDT, false>(a, s);
   }
-  const int64_t tn = cdiv(a.N, BN);
-  const unsigned grid = (unsigned)((cdiv(a.T, BM) + a.E) * tn);
-  // whole 32-element vector loads where rows and K steps are aligned
-  const auto k = rows16 && a.K % BK == 0 ? k_grouped_gemm_f16<ADT, BDT, true> : k_grouped_gemm_f16<ADT, BDT, false>;
-  hipLaunchKernelGGL(k, grid, kThreads, 0, s, a.A, a.lda, a.B, a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C,
-                     a.ldc, (uint32_t)tn);
 }
 
 template <int ADT>
@@ -448,7 +325,7 @@ int cin_grouped_gemm_f16(const void* A, int a_dtype, int64_t lda, const void* B,
   if (E == 0 || T == 0 || N == 0) return CIN_OK;
   CIN_CHECK_ARG(A && B && starts && ends && C, "grouped_gemm_f16: null pointer");
   CIN_CHECK_ARG(lda >= K && ldb >= K && ldc >= N && sbe >= 0, "grouped_gemm_f16: bad strides");
-  CIN_CHECK_ARG((cdiv(T, BM) + E) * cdiv(N, BN) < ((int64_t)1 << 31), "grouped_gemm_f16: grid too large");
+  CIN_CHECK_ARG((cdiv(T, 128) + E) * cdiv(N, 128) < ((int64_t)1 << 31), "grouped_gemm_f16: grid too large");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Args a = {A, lda, B, sbe, ldb, starts, ends, E, T, N, K, static_cast<_Float16*>(C), ldc};
   if (a_dtype == CIN_DT_BF16)

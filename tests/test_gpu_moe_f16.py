@@ -53,13 +53,14 @@ def test_grouped_f16_parity(kern, dev, xdt, wdt, N, K):
     assert (got - want).abs().max() / want.abs().max() <= 1e-3
 
 
-# Every tile of the aligned path (64 x 128, 128 x 128, 256 x 256): partial rows, columns and K
-# steps, one K step, experts without rows, more than 64 experts; and against the general kernel
-# (unaligned rows), whose sums it repeats in the same order
+# Every tile (64 x 128, 128 x 128, 256 x 256): partial rows, columns and K steps, one K step,
+# experts without rows, more than 64 experts, odd K; and against rows that start anywhere
+# (loaded without alignment), whose sums are the same in the same order
 @pytest.mark.parametrize("counts,N,K", [
     ([3, 0, 65, 1, 40], 136, 8), ([2] * 66 + [0, 100], 200, 200),
     ([300, 0, 128, 1, 555, 64, 0, 1000], 328, 520),
     ([9000, 0, 257, 7127, 1], 2120, 72),
+    ([300, 0, 70, 5], 100, 131), ([2] * 66 + [100], 64, 7), ([700, 300], 130, 1),
 ])
 @pytest.mark.parametrize("xdt,wdt", [(torch.bfloat16, torch.float32), (torch.float16, torch.bfloat16),
                                      (torch.float32, torch.float16)])
