@@ -113,10 +113,11 @@ __device__ __forceinline__ void store4(void* C, int64_t off, int c_dtype, const 
   }
 }
 
-// TAIL: K % 128 != 0, the last block's chunks past K read as zero.
+// TAIL: K % 128 != 0, the last block's chunks past K read as zero.  With one group the sums start at
+// K block kb0 and wrap around (see grouped_first_block in gemm.hip).
 template <class C, bool TAIL>
 __device__ __forceinline__ void tile(const Tile& t, int64_t lda, int64_t ssam, int64_t ssak, int64_t ldb,
-                                     int64_t ssbk, int K, int c_dtype, int64_t ldc, uint8_t* smem) {
+                                     int64_t ssbk, int K, int c_dtype, int64_t ldc, uint8_t* smem, int kb0 = 0) {
   constexpr int WN = C::WN, MT = C::MT, NT = C::NT, KS = C::KS;
   const int lane = threadIdx.x & 63;
   const int wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -137,9 +138,13 @@ __device__ __forceinline__ void tile(const Tile& t, int64_t lda, int64_t ssam, i
   const uint32_t ssak4 = (uint32_t)(ssak * 4);
   const uint32_t lds0 = (uint32_t)(uintptr_t)smem + (uint32_t)(grp * C::kBlock + wave * 1024);
   const uint32_t lds0s = (uint32_t)(uintptr_t)smem + (uint32_t)(grp * C::kBlock + C::kA + C::kB + wave * 256);
+  auto block = [&](int k) {
+    if constexpr (KS > 1) return k * KS + grp;
+    return k + kb0 < nkb ? k + kb0 : k + kb0 - nkb;
+  };
   // the group's K block of iteration k; past the last block everything reads as zero
   auto dma = [&](int k, int stg) {
-    const int kb = k * KS + grp;
+    const int kb = block(k);
     const uint32_t so = (uint32_t)kb * 128u;
     uint32_t out = 0;
     if constexpr (TAIL || KS > 1) out = kb * 128 + ch * 16 < K ? 0u : kOut;
@@ -166,7 +171,7 @@ __device__ __forceinline__ void tile(const Tile& t, int64_t lda, int64_t ssam, i
   // the B scales of 64 iterations, one per lane (zero past the last block): a scale loaded
   // where it is used would put its latency into every iteration
   auto load_sb = [&](int k) {
-    const int kb = (k + lane) * KS + grp;
+    const int kb = block(k + lane);
     return kb < nkb ? t.sb[(int64_t)kb * ssbk] : 0.0f;
   };
   v4f acc[MT][NT];

@@ -1613,14 +1613,48 @@ __global__ __launch_bounds__(C::kThreads) void k_gemm_fp8_bs_tile(
   gt::tile<C, TAIL>(t, lda, ssam, ssak, ldb, ssbk, K, c_dtype, ldc, smem);
 }
 
-// Grouped products on the same tiles.
+// The K block at which the persistent grouped walk on G workgroups (pers::GroupedSrc) starts the
+// sums of row `row` of expert e's range at columns n0 ..: nk / 8 blocks further on for each XCD.
+// Its 256 x 256 tiles and the smaller ones thus add a product's blocks in the same order: which
+// of them a number of rows gets does not move a bit of the result.  Lane l of each wave looks
+// at experts l, l + 64, ...
+__device__ inline int grouped_first_block(const int64_t* __restrict__ starts, const int64_t* __restrict__ ends,
+                                          int64_t E, int64_t Tn, int64_t e, int64_t row, int64_t n0, int64_t N,
+                                          uint32_t G, int nk) {
+  if (nk < 16) return 0;
+  int total = 0, before = 0;  // 256-row tiles: of all experts, of those before e
+  for (int64_t x = threadIdx.x & 63; x < E; x += 64) {
+    int64_t s0, s1;
+    clamp_range(starts, ends, x, Tn, s0, s1);
+    const int n = (int)((s1 - s0 + big::TM - 1) / big::TM);
+    total += n;
+    before += x < e ? n : 0;
+  }
+#pragma unroll
+  for (int d = 32; d >= 1; d >>= 1) {
+    total += __shfl_xor(total, d, 64);
+    before += __shfl_xor(before, d, 64);
+  }
+  int64_t s0, s1;
+  clamp_range(starts, ends, e, Tn, s0, s1);
+  // the walk index of that tile (big::raster<8>), and the XCD of its workgroup (pers::first_tile)
+  const uint32_t gm = (uint32_t)(before + (int)((row - s0) / big::TM)), tn = (uint32_t)(n0 / big::TN);
+  const uint32_t first = gm & ~7u, left = (uint32_t)total - first;
+  const uint32_t v = first * (uint32_t)cdiv(N, big::TN) + tn * (left < 8 ? left : 8) + (gm - first);
+  const uint32_t i = v % G;
+  const uint32_t xcd = (G & 7u) ? i & 7u : i / (G >> 3);
+  return __builtin_amdgcn_readfirstlane((int)((xcd * (uint32_t)nk) >> 3));
+}
+
+// Grouped products on the same tiles.  walk: the persistent kernels' grid where those would take
+// the product too, else 0 (K blocks in order).
 template <class C, bool TAIL>
 __global__ __launch_bounds__(C::kThreads) void k_grouped_gemm_fp8_tile(
     const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ sa, int64_t ssam,
     int64_t ssak, const uint8_t* __restrict__ B, int64_t sbe, int64_t ldb,
     const float* __restrict__ sb, int64_t ssbe, int64_t ssbn, int64_t ssbk,
     const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t Tn,
-    int64_t N, int K, void* Cp, int c_dtype, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n) {
+    int64_t N, int K, void* Cp, int c_dtype, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n, uint32_t walk) {
   __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
   uint32_t tm, tn;
   big::raster<4>(big::xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
@@ -1635,7 +1669,10 @@ __global__ __launch_bounds__(C::kThreads) void k_grouped_gemm_fp8_tile(
   t.C = static_cast<uint8_t*>(Cp) + (row0 * ldc + n0) * (c_dtype == CIN_DT_F32 ? 4 : 2);
   t.rows_a = __builtin_amdgcn_readfirstlane((int)(row_end - row0 < C::TM ? row_end - row0 : C::TM));
   t.rows_b = (int)(N - n0 < C::TN ? N - n0 : C::TN);
-  gt::tile<C, TAIL>(t, lda, ssam, ssak, ldb, ssbk, K, c_dtype, ldc, smem);
+  int kb0 = 0;
+  if constexpr (C::KS == 1)
+    if (walk) kb0 = grouped_first_block(starts, ends, E, Tn, e, row0, n0, N, walk, K >> 7);
+  gt::tile<C, TAIL>(t, lda, ssam, ssak, ldb, ssbk, K, c_dtype, ldc, smem, kb0);
 }
 
 // Grouped weight gradient on the same tiles (operands and result of pers::
@@ -1869,14 +1906,17 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
   const int64_t ncu = cin_device_cus();
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool big_ok = K % big::TK == 0 && T >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak);
+  const int64_t mt = cdiv(T, big::TM) + E, mtn = mt * cdiv(N, big::TN);
+  const unsigned pers_grid = (unsigned)(mtn < ncu ? mtn : ncu);
   if (gt::offsets_fit(128, lda, ldb, K, ssam, ssak)) {
+    const uint32_t walk = big_ok && E > 1 && E <= pers::kMaxExpertsLds ? pers_grid : 0;
     const auto launch = [&](auto cfg) {
       using C_ = decltype(cfg);
       // sum over experts of ceil(rows / TM) is at most this; surplus workgroups leave at once
       const int64_t tm = cdiv(T, C_::TM) + E - 1, tn = cdiv(N, C_::TN);
       const auto k = K % 128 == 0 ? k_grouped_gemm_fp8_tile<C_, false> : k_grouped_gemm_fp8_tile<C_, true>;
       hipLaunchKernelGGL(k, (unsigned)(tm * tn), C_::kThreads, 0, s, A, lda, sa, ssam, ssak, B, sbe, ldb, sb, ssbe, ssbn,
-                         ssbk, starts, ends, E, T, N, (int)K, C, c_dtype, ldc, (uint32_t)tm, (uint32_t)tn);
+                         ssbk, starts, ends, E, T, N, (int)K, C, c_dtype, ldc, (uint32_t)tm, (uint32_t)tn, walk);
     };
     CIN_CHECK_ARG(big_ok || (cdiv(T, 128) + E) * cdiv(N, 128) < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
     if (E == 1) {
@@ -1908,13 +1948,11 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
     }
   }
   if (big_ok) {
-    const int64_t mt = cdiv(T, big::TM) + E;
     const uint32_t tn = (uint32_t)cdiv(N, big::TN);
-    CIN_CHECK_ARG(mt * tn < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
+    CIN_CHECK_ARG(mtn < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
     if (E <= pers::kMaxExpertsLds) {
-      const unsigned grid = (unsigned)(mt * tn < ncu ? mt * tn : ncu);
 #define CIN_LAUNCH_GROUPED_PERS(EPI_)                                                                \
-  hipLaunchKernelGGL(pers::k_grouped_gemm_fp8_pers<EPI_>, grid, big::kThreads, 0,                      \
+  hipLaunchKernelGGL(pers::k_grouped_gemm_fp8_pers<EPI_>, pers_grid, big::kThreads, 0,                      \
                      static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, sbe, ldb, sb, ssbe, ssbn, \
                      ssbk, starts, ends, (int)E, T, N, K, C, c_dtype, ldc, tn)
       const int epi = pers_epi(c_dtype, C, ldc, 0);
@@ -1929,7 +1967,7 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
 #undef CIN_LAUNCH_GROUPED_PERS
       return cin_check_launch("grouped_gemm_fp8");
     }
-    hipLaunchKernelGGL(big::k_grouped_gemm_fp8_256, (unsigned)(mt * tn), big::kThreads, 0,
+    hipLaunchKernelGGL(big::k_grouped_gemm_fp8_256, (unsigned)mtn, big::kThreads, 0,
                        static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, sbe, ldb, sb,
                        ssbe, ssbn, ssbk, starts, ends, E, T, N, K, C, c_dtype, ldc, tn,
                        (uint32_t)mt);

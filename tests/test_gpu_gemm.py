@@ -309,6 +309,60 @@ def test_grouped_tile_edges(kern, dev, counts, N, K):
     assert torch.equal(y16.cpu(), y32.cpu().to(torch.bfloat16)), "bf16 output is not RNE(fp32 output)"
 
 
+def _walk_order_ref(codes, sa, w, sb, counts, N, grid):
+    """The grouped product bit for bit, its K blocks added in the order of the persistent walk:
+    walk index v of the 256 x 256 tiles (groups of 8 row tiles, column by column) belongs to
+    workgroup v % grid, and the sums on XCD x start x / 8 of the way into K.  The blocks'
+    products are whole numbers and thus exact in any order; each joins the sum by one fma."""
+    nk, tiles_n = codes.shape[1] // 128, -(-N // 256)
+    tiles, row = [], 0  # (expert, first row, end) of every row tile
+    for e, c in enumerate(counts):
+        tiles += [(e, row + r, min(row + r + 256, row + c)) for r in range(0, c, 256)]
+        row += c
+    out = torch.empty(row, N)
+    for v in range(len(tiles) * tiles_n):
+        first = v // (8 * tiles_n) * 8
+        gm = min(8, len(tiles) - first)
+        e, r0, r1 = tiles[first + (v - first * tiles_n) % gm]
+        n0 = (v - first * tiles_n) // gm * 256
+        n1 = min(n0 + 256, N)
+        i = v % grid
+        xcd = i % 8 if grid % 8 else i // (grid // 8)
+        kb0 = xcd * nk // 8 if nk >= 16 else 0
+        acc = torch.zeros(r1 - r0, n1 - n0)
+        for kb in [*range(kb0, nk), *range(kb0)]:
+            k = slice(kb * 128, kb * 128 + 128)
+            p = codes[r0:r1, k].double() @ w[e, n0:n1, k].double().t()
+            c = sa[r0:r1, kb, None] * sb[e, n0 // 128:-(-n1 // 128), kb].repeat_interleave(128)[None, :n1 - n0]
+            acc = (p * c.double() + acc.double()).float()
+        out[r0:r1, n0:n1] = acc
+    return out
+
+
+# 32- and 64-row tiles, and the 256-row ones whose order they follow: fewer workgroups than CUs
+# (a multiple of 8 and not), a full grid, shifted last columns, no rotation below 16 K blocks
+@pytest.mark.parametrize("counts,N,K", [
+    ([3, 0, 33, 1, 64, 20, 0, 141], 512, 2176), ([20] * 14 + [1, 2], 384, 2048), ([70, 20, 1, 300], 640, 4224),
+    ([5, 0, 280, 30] * 4 + [0] * 80, 768, 2048), ([9] * 40, 2048, 2048), ([40, 0, 30, 200], 512, 1920),
+    ([300, 700, 0, 128], 640, 2176),
+])
+def test_grouped_sums_do_not_depend_on_the_tile(kern, dev, counts, N, K):
+    from cinnamon_amd import layers
+    g = torch.Generator().manual_seed(K + len(counts))
+    T, E, nk = sum(counts), len(counts), K // 128
+    codes = torch.randint(-2, 3, (T, K), generator=g).float()
+    w = torch.randint(-2, 3, (E, N, K), generator=g).float()
+    sa = torch.rand(T, nk, generator=g) + 0.5
+    sb = torch.rand(E, -(-N // 128), nk, generator=g) + 0.5
+    ends = torch.tensor(counts).cumsum(0)
+    out = layers.fp8_grouped_gemm(
+        codes.to(torch.float8_e4m3fn).to(dev), sa.to(dev), w.to(torch.float8_e4m3fn).view(torch.uint8).to(dev),
+        sb.to(dev), (ends - torch.tensor(counts)).to(dev), ends.to(dev), out_dtype=torch.float32)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    grid = min((-(-T // 256) + E) * -(-N // 256), cus)
+    assert torch.equal(out.cpu(), _walk_order_ref(codes, sa, w, sb, counts, N, grid))
+
+
 def test_grouped_equals_dense_for_one_expert(kern, dev):
     from cinnamon_amd import layers
     xq, xs, wq, ws, starts, ends = _grouped_case([1000], 256, 384, seed=21)
