@@ -32,7 +32,6 @@ kernels.
 from __future__ import annotations
 
 import torch
-from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib
 from ._lib import call, dtype_code, ptr, stream_of
@@ -77,16 +76,28 @@ def custom_op(name: str, schema: str):
     return deco
 
 
-def _plain_eager(*tensors) -> bool:
-    """True outside tracing: no torch.compile, no dispatch mode (FakeTensor, make_fx,
-    functionalization), no functorch transform, and plain tensors (or, where no graph is
-    recorded, parameters: the autograd Functions are handed the layers' own)."""
-    if (torch.compiler.is_compiling() or _get_current_dispatch_mode() is not None
-            or torch._C._are_functorch_transforms_active()):
+# What a direct launch must not be hidden from, bound once (each attribute lookup on torch._C
+# costs as much as the call): these are asked on every launch.
+_dispatch_modes = torch._C._len_torch_dispatch_stack
+_function_mode = torch._C._is_torch_function_mode_enabled
+_functorch = torch._C._are_functorch_transforms_active
+_jit_tracing = torch._C._is_tracing
+_profiling = torch._C._autograd._profiler_enabled
+_grad_enabled = torch.is_grad_enabled
+_VALUES = frozenset((int, bool, float, type(None), torch.dtype))
+
+
+def _plain_eager(*args) -> bool:
+    """True where nothing but the result of a call matters: no torch.compile, no jit trace, no
+    profiler, no dispatch mode (FakeTensor, make_fx, functionalization) or function mode, no
+    functorch transform; and every argument is a plain tensor (or, where no graph is recorded, a
+    parameter: the autograd Functions are handed the layers' own) or a plain value."""
+    if (torch.compiler.is_compiling() or _dispatch_modes() or _functorch() or _function_mode() or _jit_tracing()
+            or _profiling()):
         return False
-    for t in tensors:
-        c = type(t)
-        if c is not torch.Tensor and not (c is torch.nn.Parameter and not torch.is_grad_enabled()):
+    for a in args:
+        c = type(a)
+        if c is not torch.Tensor and c not in _VALUES and not (c is torch.nn.Parameter and not _grad_enabled()):
             return False
     return True
 
@@ -96,20 +107,17 @@ def _run(op, *args):
     same kernels on the same arguments, without torch's dispatcher, whose host cost per call
     exceeds the device time of a small launch.  Only for operators without an autograd
     formula (these run inside the autograd Functions, or where no gradient is defined)."""
-    if _plain_eager(*[a for a in args if isinstance(a, torch.Tensor)]):
-        return _LAUNCH[op](*args)
-    return op(*args)
+    return _LAUNCH[op](*args) if _plain_eager(*args) else op(*args)
 
 
 def _run_detached(op, *args):
     """_run for an operator whose result could be mistaken for a differentiable one: with an
     input that records a graph, the operator runs (and refuses the backward)."""
-    tensors = [a for a in args if isinstance(a, torch.Tensor)]
-    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
-        return op(*args)
-    if _plain_eager(*tensors):
-        return _LAUNCH[op](*args)
-    return op(*args)
+    if _grad_enabled():
+        for a in args:
+            if type(a) is torch.Tensor and a.requires_grad:
+                return op(*args)
+    return _run(op, *args)
 
 
 def _require(cond: bool, msg: str) -> None:

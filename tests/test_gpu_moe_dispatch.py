@@ -358,3 +358,25 @@ def test_combine_every_top_k(dev, k, D, dtype):
     assert torch.equal(got_dy, dy)
     # D products summed in fp32 over at most D / 8 + 6 additions in a chain
     assert ((got_ds.double() - ds).abs() <= (D / 8 + 8) * 2 ** -23 * D ** 0.5 * 16).all()
+
+
+def test_traced_dispatch_computes_on_other_inputs(dev):
+    """torch.jit.trace records the operators, so the traced chain runs them on whatever it is
+    given (not the memory their outputs happened to have)."""
+    E, k, D = 8, 2, 256
+
+    def chain(x, idx, sc):
+        perm, inv, _, starts, ends = moe.moe_route(idx, E)
+        rows = x.index_select(0, torch.div(perm, k, rounding_mode="floor"))
+        return moe.moe_combine(rows, sc, inv), moe.moe_gather_sum(rows, inv, k, torch.float32), starts, ends
+
+    def inputs(seed):
+        g = torch.Generator(device=dev).manual_seed(seed)
+        x = torch.randn(40, D, generator=g, device=dev).to(torch.bfloat16)
+        idx = torch.rand(40, E, generator=g, device=dev).argsort(dim=1)[:, :k].contiguous()
+        return x, idx, torch.rand(40, k, generator=g, device=dev)
+
+    traced = torch.jit.trace(chain, inputs(1), check_trace=False)
+    for seed in (1, 2, 3):
+        for got, want in zip(traced(*inputs(seed)), chain(*inputs(seed))):
+            assert torch.equal(got, want)

@@ -261,3 +261,50 @@ def test_direct_launch_only_where_no_graph_is_recorded(monkeypatch):
         kernels._run_detached(op, plain, leaf, param)
         kernels._run(op, param)
     assert took == ["launch", "operator", "operator", "operator", "launch", "launch"]
+
+
+@kernels.custom_op("test_double", "(Tensor x) -> Tensor")
+def _double_op(x):
+    """2 x on the CPU, written where torch does not see it, as a kernel writes its output."""
+    out = torch.empty_like(x)
+    out.numpy()[...] = x.detach().numpy() * 2
+    return out
+
+
+@_double_op.register_fake
+def _(x):
+    return torch.empty_like(x)
+
+
+@pytest.mark.parametrize("run", [kernels._run, kernels._run_detached])
+def test_trace_records_the_operator(run):
+    """torch.jit.trace keeps the operator, not the allocation of its output: the traced function
+    computes on other inputs."""
+    traced = torch.jit.trace(lambda x: run(_double_op, x), (torch.ones(4),), check_trace=False)
+    assert "cinnamon_amd::test_double" in str(traced.graph)
+    x = torch.arange(4.0)
+    assert torch.equal(traced(x), 2 * x)
+
+
+@pytest.mark.parametrize("run", [kernels._run, kernels._run_detached])
+def test_modes_and_profiler_see_the_operator(run):
+    seen = []
+
+    class Watch(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    with Watch():
+        run(_double_op, torch.ones(4))
+    assert any("test_double" in s for s in seen)
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        run(_double_op, torch.ones(4))
+    assert "cinnamon_amd::test_double" in [e.key for e in prof.key_averages()]
+
+    class Other:  # a value of another library that overrides torch's functions
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return str(func)
+
+    assert "test_double" in run(_double_op, Other())
