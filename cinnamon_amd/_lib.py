@@ -147,7 +147,10 @@ def dtype_code(t) -> int:
 def stream_of(t: torch.Tensor) -> int:
     """torch's current HIP stream on the tensor's device (as a hipStream_t)."""
     # (the raw handle: torch.cuda.current_stream builds a Stream object, 2.2 us against 0.2)
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    device = t.get_device()
+    if device < 0:  # torch would read it as the current device, and the kernel host memory
+        raise ValueError(f"expected a device tensor, got one on {t.device}")
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def ptr(t: torch.Tensor | None) -> int:

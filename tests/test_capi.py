@@ -144,3 +144,15 @@ def test_moe_route_workspace_size():
     assert lib.cin_moe_route_workspace(16384, 8, 32) == 2 * 128 * 32   # 1024 assignments per block
     assert lib.cin_moe_route_workspace(1, 1, 4) == 8
     assert lib.cin_moe_route_workspace(0, 8, 4) == 0
+
+
+def test_host_tensors_have_no_stream():
+    """A tensor in host memory is refused before a launch: it has no device whose stream could
+    run a kernel on it (and the launch would hand the kernel a host address)."""
+    import torch
+
+    from cinnamon_amd import kernels  # noqa: F401  (registers the operators)
+    with pytest.raises(ValueError, match="device tensor"):
+        _lib.stream_of(torch.zeros(4))
+    with pytest.raises(ValueError, match="device tensor"):
+        torch.ops.cinnamon_amd.quant_rowwise(torch.zeros(4, 128), 128, False, False)
