@@ -434,9 +434,9 @@ def _codes_t(like, rows, cols):
     """[rows, cols] codes whose rows do not lie a multiple of 16 KiB apart: that far apart, one
     128-byte column of many rows falls on few memory channels (a wgrad over 16384 tokens, 4096
     x 1024: 92.5 us, with 256 bytes between the rows 79.2; 8192 tokens: no difference)."""
-    if cols % 16384 == 0:
-        return _codes(like, rows, cols + 256)[:, :cols]
-    return _codes(like, rows, cols)
+    # (arithmetic, not a branch: a symbolic column count must record no guard on its value)
+    gap = 256 * ((16384 - cols % 16384) // 16384)
+    return like.new_empty_strided((rows, cols), (cols + gap, 1), dtype=torch.float8_e4m3fn)
 
 
 def _launch_quant_bwd(entry, codes_t, cols_t, grad, x_fp8, x_scale, round_scale, col_scales):

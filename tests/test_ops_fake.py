@@ -308,3 +308,29 @@ def test_modes_and_profiler_see_the_operator(run):
             return str(func)
 
     assert "test_double" in run(_double_op, Other())
+
+
+@pytest.mark.parametrize("tokens", [16384, 5000])
+def test_padded_backward_quantization_records_no_guard(tokens):
+    """A symbolic token count stays symbolic through the shape functions of the backward's
+    quantizations, also where the transposed rows get a gap (whole multiples of 16 KiB): a guard
+    would compile the backward anew for other token counts."""
+    from torch._dynamo.source import ConstantSource
+    from torch.fx.experimental.symbolic_shapes import DimDynamic, ShapeEnv, StatelessSymbolicContext
+
+    env = ShapeEnv()
+    mode = FakeTensorMode(shape_env=env)
+    gy = mode.from_tensor(torch.empty(tokens, 512, dtype=BF16), source=ConstantSource("gy"), symbolic_context=(
+        StatelessSymbolicContext(dynamic_sizes=[DimDynamic.DYNAMIC, DimDynamic.STATIC], constraint_sizes=[None, None])))
+    with mode:
+        xq = gy.new_empty((gy.shape[0], 256), dtype=F8)
+        xs = gy.new_empty((gy.shape[0], 2), dtype=F32)
+        for op, args in ((kernels._quant_bwd_op, (False, True)), (kernels._quant_bwd_padded_op, (False,))):
+            outs = op(gy, xq, xs, *args)
+            assert len(outs) == 6 and [str(g.expr) for g in env.guards] == []
+
+
+@pytest.mark.parametrize("cols", [0, 128, 16256, 16384, 16512, 32768])
+def test_transposed_code_rows_lie_no_multiple_of_16_kib_apart(cols):
+    t = kernels._codes_t(torch.empty(1), 3, cols)
+    assert t.shape == (3, cols) and t.stride() == (cols + (256 if cols % 16384 == 0 else 0), 1)
