@@ -1163,8 +1163,7 @@ __device__ __forceinline__ P* uniform_ptr(P* p) {
 template <int EPI, class Src, bool VARK = false>
 __device__ __forceinline__ void run_tiles(const Src& src, int64_t lda, int64_t ssam, int64_t ssak,
                                           int64_t ldb, int64_t ssbn, int64_t ssbk, int64_t K,
-                                          int c_dtype, int64_t ldc) {
-  __shared__ SmemAll smu;
+                                          int c_dtype, int64_t ldc, SmemAll& smu) {
   Smem& sm = smu.s;
   const uint32_t G = gridDim.x;
   uint32_t v = first_tile(blockIdx.x, G);
@@ -1407,7 +1406,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_gemm_fp8_bs_pers(
   src.lda = lda; src.ssam = ssam; src.ldb = ldb; src.ssbn = ssbn; src.ldc = ldc; src.M = M; src.N = N;
   src.es = c_dtype == CIN_DT_F32 ? 4 : 2;
   src.tiles_m = tiles_m; src.tiles_n = tiles_n; src.G = gridDim.x;
-  run_tiles<EPI>(src, lda, ssam, ssak, ldb, ssbn, ssbk, K, c_dtype, ldc);
+  __shared__ SmemAll smu;
+  run_tiles<EPI>(src, lda, ssam, ssak, ldb, ssbn, ssbk, K, c_dtype, ldc, smu);
 }
 
 constexpr int kMaxExpertsLds = 4096;
@@ -1459,7 +1459,8 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_gemm_fp8_pers(
   src.lda = lda; src.ssam = ssam; src.ldb = ldb; src.sbe = sbe; src.ssbe = ssbe; src.ssbn = ssbn;
   src.ldc = ldc; src.Tn = Tn; src.N = N; src.es = c_dtype == CIN_DT_F32 ? 4 : 2;
   src.tiles_n = tiles_n; src.starts = starts; src.ends = ends; src.E = E; src.tpre = tpre;
-  run_tiles<EPI>(src, lda, ssam, ssak, ldb, ssbn, ssbk, K, c_dtype, ldc);
+  __shared__ SmemAll smu;
+  run_tiles<EPI>(src, lda, ssam, ssak, ldb, ssbn, ssbk, K, c_dtype, ldc, smu);
 }
 
 // Grouped weight gradient on the persistent walk (same operands and result as
@@ -1471,6 +1472,11 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_gemm_fp8_pers(
 // the long tiles are dealt out evenly and the static walk stays balanced.
 constexpr int kMaxWgradExperts = 512;
 static_assert(kMaxWgradExperts <= kThreads, "the wgrad's LDS tables give each thread one expert");
+
+// The tile of an expert-sorted walk: every other full round of G is taken in reverse.
+__device__ inline uint32_t snake(uint32_t i, uint32_t b, uint32_t G, uint32_t total) {
+  return (i & 1u) && (i + 1) * G <= total ? i * G + (G - 1 - b) : i * G + b;
+}
 
 struct WgradSrc {
   const uint8_t* A; const float* sa; const uint8_t* B; const float* sb; uint8_t* C;
@@ -1486,8 +1492,8 @@ struct WgradSrc {
   __device__ bool fewer(uint32_t) const { return false; }  // no start offsets (above)
   __device__ bool get(uint32_t v, Tile& t) const {
     if (v >= total) return false;
-    const uint32_t i = v / G, b = v - i * G;
-    const uint32_t u = ((i & 1u) && (i + 1) * G <= total) ? i * G + (G - 1 - b) : v;
+    const uint32_t i = v / G;
+    const uint32_t u = snake(i, v - i * G, G, total);
     const uint32_t per = tiles_m * tiles_n;
     const uint32_t rank = u / per, r = u - rank * per;
     // LDS reads are per lane to the compiler: made wave-uniform, what follows stays scalar
@@ -1513,17 +1519,30 @@ struct WgradSrc {
   }
 };
 
+// by_load: where one workgroup's share (K blocks, and kTileCost a tile for its prologue and C) is
+// over 1.6 times that of as many average tiles, the workgroups walk 128 x 128 tiles instead, a quarter of the work
+// each, that take two K blocks at once: slower work (even loads 1.2-1.6 times as long), but no
+// CU is left with most of it.  us, 256 x 256 / 128 x 128, Zipf(1.1) rows, T, E, N, K: 32768, 16, 1024,
+// 1024: 118 / 78; 32768, 16, 2048, 1024: 140 / 118; 32768, 64, 1024, 1024: 231 / 169; 131072, 32, 1024,
+// 1024: 576 / 354; 32768, 16, 2048, 2048 (a share of 1.4): 258 / 304; equal rows: 32768, 16, 1024, 1024:
+// 41 / 60.  (A launch of its own, which could put two workgroups on a CU, takes 68 in the first
+// case, but an empty launch beside it 5-8 where the loads are even.)
+constexpr int kTileCost = 10;
+using UnevenTile = gt::Cfg<2, 2, 4, 4, 2>;
+static_assert(UnevenTile::kBytes <= (int)sizeof(SmemAll) && UnevenTile::kThreads == kThreads, "share the walk's workgroups");
+
 template <int EPI>
 __global__ __launch_bounds__(kThreads, 1) void k_grouped_wgrad_fp8_pers(
     const uint8_t* __restrict__ A, int64_t lda, const float* __restrict__ sa, int64_t ssam,
     int64_t ssak, const uint8_t* __restrict__ B, int64_t ldb, const float* __restrict__ sb, int64_t ssbm,
     const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int E, int64_t Tn,
     int64_t tcap, int64_t M, int64_t N, void* C, int c_dtype, int64_t ldc, int64_t sce,
-    uint32_t tiles_m, uint32_t tiles_n) {
+    uint32_t tiles_m, uint32_t tiles_n, int by_load) {
+  __shared__ SmemAll smu;
   __shared__ int order[kMaxWgradExperts];
   __shared__ int enk[kMaxWgradExperts];
   __shared__ int64_t poff[kMaxWgradExperts];
-  __shared__ int wtot[kThreads / 64];
+  __shared__ int wtot[kThreads / 64], wmost[kThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // thread t owns expert t (E <= kThreads): K blocks, then the exclusive prefix of the
   // padded sizes 128 * nk (the padded token axis of the operands)
@@ -1579,14 +1598,71 @@ __global__ __launch_bounds__(kThreads, 1) void k_grouped_wgrad_fp8_pers(
       }
     }
   }
+  const uint32_t G = gridDim.x;
+  if (by_load && nz > 0) {
+    const uint32_t per = tiles_m * tiles_n, total = (uint32_t)nz * per;
+    int blocks = 0;
+    for (int w = 0; w < kThreads / 64; ++w) blocks += wtot[w];
+    const int64_t rounds = cdiv(total, G);
+    // 8 / 5 of a workgroup's share if every tile were an average one, times 5 nz
+    const int64_t even = 8 * rounds * (blocks + kTileCost * (int64_t)nz);
+    // (no share is longer than that many tiles of the longest kind: near even loads nothing more
+    // is looked at)
+    int most = (int)rounds * (enk[order[0]] + kTileCost);
+    if ((int64_t)most * 5 * nz > even) {
+      most = 0;
+      for (uint32_t b = tid; b < G; b += kThreads) {
+        int share = 0;
+        for (uint32_t i = 0; i * G < total; ++i) {
+          const uint32_t u = snake(i, b, G, total);
+          if (u < total) share += enk[order[u / per]] + kTileCost;
+        }
+        most = share > most ? share : most;
+      }
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) {
+        const int o = __shfl_xor(most, d, 64);
+        most = o > most ? o : most;
+      }
+      if (lane == 0) wmost[wave] = most;
+      __syncthreads();
+      for (int w = 0; w < kThreads / 64; ++w) most = wmost[w] > most ? wmost[w] : most;
+    }
+    if ((int64_t)most * 5 * nz > even) {
+      const uint32_t tm = (uint32_t)cdiv(M, UnevenTile::TM), tn = (uint32_t)cdiv(N, UnevenTile::TN);
+      const uint32_t all = (uint32_t)nz * tm * tn;
+      for (uint32_t i = 0; i * G < all; ++i) {
+        const uint32_t u = snake(i, blockIdx.x, G, all);
+        if (u >= all) break;
+        if (i) __syncthreads();  // the last tile's results have left LDS
+        const uint32_t rank = u / (tm * tn);
+        const int e = __builtin_amdgcn_readfirstlane(order[rank]);
+        const int64_t kb0 = __builtin_amdgcn_readfirstlane((int)(poff[e] >> 7));
+        uint32_t im, in;
+        raster<4>(u - rank * tm * tn, tm, tn, im, in);
+        const int64_t m0 = (int64_t)im * UnevenTile::TM, n0 = (int64_t)in * UnevenTile::TN;
+        gt::Tile t;
+        t.A = A + m0 * lda + kb0 * TK;
+        t.sa = sa + m0 * ssam + kb0 * ssak;
+        t.B = B + n0 * ldb + kb0 * TK;
+        t.sb = sb + kb0 * ssbm + (n0 >> 7);
+        t.C = static_cast<uint8_t*>(C) + ((int64_t)e * sce + m0 * ldc + n0) * (c_dtype == CIN_DT_F32 ? 4 : 2);
+        t.rows_a = (int)(M - m0 < UnevenTile::TM ? M - m0 : UnevenTile::TM);
+        t.rows_b = (int)(N - n0 < UnevenTile::TN ? N - n0 : UnevenTile::TN);
+        gt::tile<UnevenTile, false>(t, lda, ssam, ssak, ldb, ssbm, __builtin_amdgcn_readfirstlane(enk[e]) * TK, c_dtype,
+                                    ldc, smu.c);
+      }
+      return;
+    }
+  }
   WgradSrc src;
   src.A = A; src.sa = sa; src.B = B; src.sb = sb; src.C = static_cast<uint8_t*>(C);
   src.lda = lda; src.ssam = ssam; src.ssak = ssak; src.ldb = ldb; src.ssbm = ssbm; src.ldc = ldc; src.sce = sce;
   src.M = M; src.N = N; src.es = c_dtype == CIN_DT_F32 ? 4 : 2;
-  src.tiles_m = tiles_m; src.tiles_n = tiles_n; src.G = gridDim.x;
+  src.tiles_m = tiles_m; src.tiles_n = tiles_n; src.G = G;
   src.total = (uint32_t)nz * tiles_m * tiles_n;
   src.order = order; src.enk = enk; src.poff = poff;
-  run_tiles<EPI, WgradSrc, true>(src, lda, ssam, ssak, ldb, 1, ssbm, 0, c_dtype, ldc);
+  run_tiles<EPI, WgradSrc, true>(src, lda, ssam, ssak, ldb, 1, ssbm, 0, c_dtype, ldc, smu);
 }
 
 }  // namespace pers
@@ -2008,13 +2084,13 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
   const int64_t tm = cdiv(N, big::TM), tn = cdiv(K, big::TN);
   CIN_CHECK_ARG(E * tm * tn < ((int64_t)1 << 31), "grouped_wgrad_fp8: grid too large");
   const int64_t cus = cin_device_cus();
-  // Up to four rounds of 256 x 256 tiles: ragged experts leave the persistent walk waiting for
-  // the CUs that hold the longest tiles (and half-filled rounds), where the 128 x 128 tiles'
-  // dispatch evens them out.  us, persistent / 128 x 128, Zipf(1.1) rows, T, E, N, K: 32768, 16,
-  // 1024, 1024 (1 round) 109 / 61; 32768, 16, 2048, 1024 (2) 135 / 95; 32768, 16, 2048, 2048 (4) 251 /
-  // 232; 65536, 32, 2048, 2048 (8) 426 / 456.
-  if ((E == 1 ? rounds_sparse(tm * tn, cus) : E * tm * tn <= 4 * cus) &&
-      gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak)) {
+  // Up to half a round of 256 x 256 tiles the 128 x 128 ones finish first whatever the loads (us,
+  // persistent / 128 x 128, T, E, N, K, equal loads: 32768, 8, 1024, 1024: 65 / 46; 2048, 32, 512, 512:
+  // 18 / 12); with up to four rounds the persistent kernel looks at the loads.
+  const int64_t tiles = E * tm * tn;
+  const bool tiles_fit = gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak);
+  const int by_load = tiles_fit && tiles <= 4 * cus && T >= 256 * E;
+  if (tiles_fit && (E == 1 ? rounds_sparse(tiles, cus) : 2 * tiles <= cus)) {
     const auto launch = [&](auto cfg) {
       using C_ = decltype(cfg);
       const uint32_t tm_ = (uint32_t)cdiv(N, C_::TM), tn_ = (uint32_t)cdiv(K, C_::TN);
@@ -2036,7 +2112,7 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
 #define CIN_LAUNCH_WGRAD_PERS(EPI_)                                                                   \
   hipLaunchKernelGGL(pers::k_grouped_wgrad_fp8_pers<EPI_>, ncu, big::kThreads, 0,                       \
                      static_cast<hipStream_t>(stream), A, lda, sa, ssam, ssak, B, ldb, sb, ssbm, starts,   \
-                     ends, (int)E, T, tcap, N, K, C, c_dtype, ldc, sce, (uint32_t)tm, (uint32_t)tn)
+                     ends, (int)E, T, tcap, N, K, C, c_dtype, ldc, sce, (uint32_t)tm, (uint32_t)tn, by_load)
     const int epi = pers_epi(c_dtype, C, ldc, sce);
     if (epi == pers::kEpiCounted16x4)
       CIN_LAUNCH_WGRAD_PERS(pers::kEpiCounted16x4);

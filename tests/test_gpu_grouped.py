@@ -505,3 +505,80 @@ def test_grouped_wgrad_persistent_direct_epilogue(kern, dev, out_dtype):
 def test_grouped_forward_many_experts_long(kern, dev, E, T):
     """The same with enough rows an expert for the 256-row tiles."""
     test_grouped_forward_many_experts(kern, dev, E, T)
+
+
+def _wgrad_order_ref(a, sa, b, sb, counts, N, K, cus):
+    """The wgrad bit for bit, and whether its loads are uneven.  The tiles of the experts with
+    tokens, longest first, are dealt to one workgroup per CU, every other full round backwards.
+    Even loads: 256 x 256 tiles, whose sums on XCD x start x / 8 of the way into the K blocks.
+    Uneven: 128 x 128 tiles that sum the even and the odd blocks apart.  The blocks' products are
+    whole numbers and exact in any order; each joins the sum by one fma."""
+    nk = [-(-c // 128) for c in counts]
+    first = [sum(nk[:e]) for e in range(len(nk))]
+    order = sorted((e for e in range(len(nk)) if nk[e]), key=lambda e: (-nk[e], e))
+    tm, tn = -(-N // 256), -(-K // 256)
+    total = len(order) * tm * tn
+
+    def walk(i, w):
+        return i * cus + cus - 1 - w if i % 2 and (i + 1) * cus <= total else i * cus + w
+
+    shares = [sum(nk[order[walk(i, w) // (tm * tn)]] + 10 for i in range(-(-total // cus)) if walk(i, w) < total)
+              for w in range(cus)]
+    uneven = (total <= 4 * cus and sum(counts) >= 256 * len(nk)
+              and max(shares) * 5 * len(order) > 8 * -(-total // cus) * (sum(nk) + 10 * len(order)))
+    out = torch.zeros(len(nk), N, K, device=a.device)
+
+    def add(acc, e, kb, n, k):
+        p = a[n, kb * 128:kb * 128 + 128].double() @ b[k, kb * 128:kb * 128 + 128].double().t()
+        c = sa[n, kb, None] * sb[kb].repeat_interleave(128)[None, k]
+        return (p * c.double() + acc.double()).float()
+
+    if uneven:
+        for e in order:
+            half = [torch.zeros(N, K, device=a.device) for _ in range(2)]
+            for i in range(nk[e]):
+                half[i % 2] = add(half[i % 2], e, first[e] + i, slice(0, N), slice(0, K))
+            out[e] = half[0] + half[1]
+        return out, uneven
+    for v in range(total):
+        i, w = divmod(v, cus)
+        rank, r = divmod(walk(i, w), tm * tn)
+        e = order[rank]
+        g = r // (4 * tn) * 4
+        gm = min(4, tm - g)
+        m0, n0 = (g + (r - g * tn) % gm) * 256, (r - g * tn) // gm * 256
+        n, k = slice(m0, min(m0 + 256, N)), slice(n0, min(n0 + 256, K))
+        xcd = w // (cus // 8) if cus % 8 == 0 else w % 8
+        kb0 = xcd * nk[e] // 8 if nk[e] >= 16 else 0
+        acc = torch.zeros(n.stop - n.start, k.stop - k.start, device=a.device)
+        for kb in [*range(kb0, nk[e]), *range(kb0)]:
+            acc = add(acc, e, first[e] + kb, n, k)
+        out[e, n, k] = acc
+    return out, uneven
+
+
+# Between half a round of 256 x 256 tiles and four: equal loads (also in a last round that is not
+# full), one expert with most of the rows, experts without any, more than 64 experts, partial tiles
+@pytest.mark.parametrize("counts,N,K,want_uneven", [
+    ([2100] * 9, 1024, 1024, False), ([2100, 2000, 2200, 1900] * 5, 1000, 1024, False),
+    ([9000, 300, 0, 40, 1, 200, 128, 129, 2000, 77], 1000, 1152, True), ([0, 0, 20000] + [1] * 7, 1024, 1024, True),
+    ([9000] + [200] * 79, 512, 384, True), ([9000, 9000, 0, 0], 1500, 2048, False), ([300] * 8 + [7000], 2048, 1024, True),
+])
+def test_grouped_wgrad_follows_the_loads(kern, dev, counts, N, K, want_uneven):
+    from cinnamon_amd import layers
+    g = torch.Generator(device=dev).manual_seed(N + len(counts))
+    T, E = sum(counts), len(counts)
+    cap = layers.padded_capacity(T, E)
+    a = torch.randint(-2, 3, (N, cap), generator=g, device=dev).float()
+    b = torch.randint(-2, 3, (K, cap), generator=g, device=dev).float()
+    sa = torch.rand(N, cap // 128, generator=g, device=dev) + 0.5
+    sb = torch.rand(cap // 128, K // 128, generator=g, device=dev) + 0.5
+    starts, ends = (t.to(dev) for t in _ranges(counts))
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    want, uneven = _wgrad_order_ref(a, sa, b, sb, counts, N, K, cus)
+    if cus == 256:
+        assert uneven == want_uneven
+    f8 = torch.float8_e4m3fn
+    for dtype in (torch.float32, torch.bfloat16):
+        got = layers.fp8_grouped_wgrad(a.to(f8), sa, b.to(f8), sb, starts, ends, T, out_dtype=dtype)
+        assert torch.equal(got, want.to(dtype))
