@@ -999,10 +999,13 @@ int cin_indexer_scores_fp8(const uint8_t* q8, const float* q_scale, const uint8_
     launch_indexer<32 * n, hg>(grid, st, q8, q_scale, k8, k_scale, weights, L, S, H,            \
                                softmax_scale, scores, tiles_t, tiles_s, xcd_rotate, vec, kpw);  \
     break;
-  if (d <= 128 && H > 4) {
-    // eight heads' fragments at once: with four, every 128-key sub-tile loaded each group's q
-    // again (16 x 1024 tokens, 8 heads, d 128: 63.7 -> 46.7 us with the quantization; 1 x 2048
-    // tokens, 8 heads, d 128: 38.7 -> 19.0 with shorter key ranges too)
+  // Eight heads' fragments at once: up to eight heads, whose q is then loaded once (with four at a
+  // time, every 128-key sub-tile loaded each group's q again: 16 x 1024 tokens, 8 heads, d 128: 44.6
+  // -> 28.2 us; 1 x 2048 tokens: 33.8 -> 15.0 with shorter key ranges too).  With more heads they are
+  // loaded again either way and the smaller group is faster (16 x 1024 tokens, d 128, 9 / 12 / 16 heads:
+  // 42.8 / 47.9 / 70.8 us, eight at a time 50.3 / 60.1 / 84.1), but for up to 16 tokens, where one wave in
+  // four has any, if eight at a time pad no further (64 x 1 tokens, 16 heads: 41.6 -> 36.7 us).
+  if (d <= 128 && H > 4 && (H <= 8 || (L <= 16 && cdiv(H, 8) * 2 == cdiv(H, 4)))) {
     switch (d / 32) {
       CIN_INDEXER_CASE(1, 8) CIN_INDEXER_CASE(2, 8) CIN_INDEXER_CASE(3, 8) CIN_INDEXER_CASE(4, 8)
     }

@@ -221,6 +221,10 @@ def test_fused_q_quantization_equals_the_two_calls_full_grid(dev, B, L, S, H, d,
     (1, 70, 1100, 5, 128, torch.bfloat16), (2, 64, 300, 8, 32, torch.float32), (1, 33, 700, 9, 96, torch.float16),
     (1, 20, 1500, 16, 64, torch.bfloat16), (9, 300, 900, 8, 64, torch.bfloat16), (20, 500, 520, 6, 32, torch.bfloat16),
     (3, 129, 513, 3, 160, torch.bfloat16),
+    # more than eight heads: eight at a time for up to 16 tokens, four for more (the cases above) and
+    # where eight would pad further
+    (5, 1, 700, 16, 64, torch.bfloat16), (2, 16, 300, 13, 32, torch.float16), (3, 9, 520, 12, 128, torch.bfloat16),
+    (2, 17, 300, 24, 64, torch.bfloat16),
 ])
 def test_scores_of_many_heads(dev, B, L, S, H, d, dtype):
     test_scores_match_the_oracle(dev, B, L, S, H, d, dtype)
