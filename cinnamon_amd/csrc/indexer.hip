@@ -889,12 +889,15 @@ __global__ void k_indexer_wgrad_finish(const float* __restrict__ partial, const 
 }
 
 // Keys per workgroup of the 4-wave scoring kernels: kKPW, or a half or a quarter of it where
-// that many leave CUs without a workgroup.  B, L, S, H, d: 2, 777, 4100, 8, 64: 512 keys (234
-// workgroups) 28.0 us, 256 keys (442) 24.4, 128 keys (858) 30.8; 1, 512, 4096, 16, 64: 56.3, 128
-// keys 21.6; 2, 300, 3000, 2, 192: 23.7, 15.4.
-int64_t keys_per_workgroup(int64_t token_tiles, int64_t S) {
+// that many leave CUs without a workgroup (past d = 128, where a workgroup loads twice the q for
+// its keys, more than a quarter of them).  B, L, S, H, d: 2, 777, 4100, 8, 64: 512 keys (234 workgroups) 28.0 us,
+// 256 keys (442) 24.4, 128 keys (858) 30.8; 1, 512, 4096, 16, 64: 56.3, 128 keys 21.6; 2, 300, 3000, 2,
+// 192: 23.7, 15.4; 1, 2048, 2048, 2, 192: 512 keys (128) 15.6, 256 keys 10.8; 2, 777, 4100, 2, 192: 512
+// keys (234) 17.0, 256 keys 18.3, quantizing q itself 19.8 and 24.4.
+int64_t keys_per_workgroup(int64_t token_tiles, int64_t S, int64_t d) {
+  const int64_t enough = d <= 128 ? cin_device_cus() : cin_device_cus() * 3 / 4;
   int64_t kpw = kKPW;
-  while (kpw > kKT && token_tiles * cdiv(S, kpw) < cin_device_cus()) kpw /= 2;
+  while (kpw > kKT && token_tiles * cdiv(S, kpw) < enough) kpw /= 2;
   return kpw;
 }
 
@@ -971,7 +974,7 @@ int cin_indexer_scores_fp8(const uint8_t* q8, const float* q_scale, const uint8_
   CIN_CHECK_ARG(q8 && q_scale && k8 && k_scale && weights && scores, "indexer_scores_fp8: null pointer");
   CIN_CHECK_ARG((((uintptr_t)q8) & 15) == 0 && (((uintptr_t)k8) & 15) == 0,
                 "indexer_scores_fp8: code buffers must be 16-byte aligned");
-  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S), tiles_s = cdiv(S, kpw);
+  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S, d), tiles_s = cdiv(S, kpw);
   CIN_CHECK_ARG(B * tiles_t * tiles_s < ((int64_t)1 << 31), "indexer_scores_fp8: grid too large");
   const unsigned grid = (unsigned)(B * tiles_t * tiles_s);
   const int xcd_rotate = grid % 8 == 0;
@@ -1065,7 +1068,7 @@ int cin_indexer_scores_fp8_q(const void* q, int q_dtype, const uint8_t* k8, cons
     }
     return cin_check_launch("indexer_scores_fp8_q");
   }
-  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S), tiles_s = cdiv(S, kpw);
+  const int64_t tiles_t = cdiv(L, kTT), kpw = keys_per_workgroup(B * tiles_t, S, d), tiles_s = cdiv(S, kpw);
   CIN_CHECK_ARG(B * tiles_t * tiles_s < ((int64_t)1 << 31), "indexer_scores_fp8_q: grid too large");
   const unsigned grid = (unsigned)(B * tiles_t * tiles_s);
   const int xcd_rotate = grid % 8 == 0;
