@@ -416,7 +416,9 @@ def test_backward_padded_equals_unpadded(kern, dev, M, N, K, dtype):
 
 # whole, partial and single-byte tiles; rows that start on any byte
 @pytest.mark.parametrize("R,C,off", [(1, 1, 0), (7, 130, 0), (128, 128, 0), (129, 1500, 3), (4000, 1500, 0),
-                                     (64, 4097, 1), (272, 136, 8)])
+                                     (64, 4097, 1), (272, 136, 8),
+                                     # every length of a row's last piece, input rows cut at every byte of one
+                                     *[(128 + n, 136 + n, 0) for n in range(1, 16)], (15, 7, 2), (33, 9, 0)])
 def test_transpose_bytes(kern, dev, R, C, off):
     g = torch.Generator().manual_seed(R + C)
     src = torch.randint(0, 256, (R, C + off), generator=g, dtype=torch.uint8).to(dev)[:, off:]
