@@ -321,20 +321,20 @@ __device__ __forceinline__ float piece_elem(const uint4 (&q)[W], int e) {
   }
 }
 
-// W 16-byte pieces, PS pieces apart, of G of a token's rows, pos[j0] .. pos[j0 + G - 1], at byte
+// W 16-byte pieces, ps pieces apart, of G of a token's rows, pos[j0] .. pos[j0 + G - 1], at byte
 // `cb` of each row (rows `rb` bytes apart), every load issued before any result is used: one
 // wave keeps G W loads in flight instead of one.  Rows at or past n load row pos[j0] again
 // (j0 < n); their pieces are never used.  Needs 16-byte aligned pieces.
-template <int G, int W, int PS, int KM>
+template <int G, int W, int KM>
 __device__ __forceinline__ void load_rows(const void* base, int64_t cb, int64_t rb,
                                           const int32_t (&pos)[KM], int j0, int n,
-                                          uint4 (&raw)[G][W]) {
+                                          uint4 (&raw)[G][W], int ps = 1) {
 #pragma unroll
   for (int jj = 0; jj < G; ++jj) {
     const int64_t r = j0 + jj < n ? pos[j0 + jj] : pos[j0];
     const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(base) + r * rb + cb);
 #pragma unroll
-    for (int u = 0; u < W; ++u) raw[jj][u] = p[u * PS];
+    for (int u = 0; u < W; ++u) raw[jj][u] = p[u * ps];
   }
 }
 
@@ -400,6 +400,8 @@ __device__ __forceinline__ void store_piece(void* base, int64_t off, int64_t nv,
 // positions and loading 8 rows for k = 2 held the wave to 2 per SIMD.  Combine / gather sum in
 // us, before and after: 16384 tokens, k 2, 1024 fp16 columns, 55.5 / 39.4 and 29.9 / 17.0 (4.5 and
 // 5.9 TB/s); 16384, k 8, 7168, 520 / 433 and 427 / 402; 64, k 8, 7168, 22.8 / 16.9 and 11.0 / 10.2.
+// Each of a lane's two pieces is loaded with the others' if it is whole; where only both together
+// were, the last step of most widths went row by row: 16384, k 8, 768 fp16 53.7 / 47.5, so 39.9 / 35.4.
 template <int GT, int OT, int KM, bool WEIGHTED>
 __device__ __forceinline__ void sum_rows(const void* __restrict__ g, int64_t sgm, const int32_t (&pos)[KM], int n,
                                          const float (&w)[KM], int64_t t, int ch, int nch, int64_t N,
@@ -407,20 +409,22 @@ __device__ __forceinline__ void sum_rows(const void* __restrict__ g, int64_t sgm
   constexpr int RB = KM < kRowBatch ? KM : kRowBatch;
   constexpr int E = kPiece<GT>, ES = GT == CIN_DT_F32 ? 4 : 2;
   const int lane = threadIdx.x & 63;
-  // whole steps of rows whose pieces are 16-byte aligned take the batched loads
+  // rows whose pieces are 16-byte aligned take the batched loads for every whole piece
   const bool vec = ((((uintptr_t)g) & 15) == 0) && ((sgm * ES) & 15) == 0;
   for (int64_t c = (int64_t)(ch * 128 + lane) * E; c < N; c += (int64_t)nch * 128 * E) {
+    const bool whole[2] = {vec && c + E <= N, vec && c + 65 * E <= N};
     float acc[2][E];
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int e = 0; e < E; ++e) acc[u][e] = 0.0f;
-    if (vec && c + 65 * E <= N) {
+    if (whole[0]) {
 #pragma unroll
       for (int j0 = 0; j0 < KM; j0 += RB) {
         if (j0 < n) {
           uint4 raw[RB][2];
-          load_rows<RB, 2, 64>(g, c * ES, sgm * ES, pos, j0, n, raw);
+          // (a second piece that is not whole: the first one again)
+          load_rows<RB, 2>(g, c * ES, sgm * ES, pos, j0, n, raw, whole[1] ? 64 : 0);
 #pragma unroll
           for (int jj = 0; jj < RB; ++jj)
             if (j0 + jj < n)
@@ -435,14 +439,22 @@ __device__ __forceinline__ void sum_rows(const void* __restrict__ g, int64_t sgm
               }
         }
       }
-    } else {
+    }
+    // pieces that the edge cuts or that are not aligned
+    const int64_t left[2] = {whole[0] ? 0 : N - c, whole[1] ? 0 : N - c - 64 * E};
+    if (left[0] > 0 || left[1] > 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[u][e] = left[u] > 0 ? 0.0f : acc[u][e];
 #pragma unroll
       for (int j = 0; j < KM; ++j) {
         if (j < n) {
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
+            if (left[u] <= 0) continue;
             float v[E];
-            load_piece<GT>(g, (int64_t)pos[j] * sgm + c + 64 * E * u, N - c - 64 * E * u, v);
+            load_piece<GT>(g, (int64_t)pos[j] * sgm + c + 64 * E * u, left[u], v);
 #pragma unroll
             for (int e = 0; e < E; ++e) acc[u][e] = acc[u][e] + (WEIGHTED ? v[e] * w[j] : v[e]);
           }
@@ -527,7 +539,7 @@ __global__ __launch_bounds__(kRT) void k_moe_combine_bwd_tokens(
         for (int j0 = 0; j0 < KM; j0 += RB) {
           if (j0 < n) {
             uint4 raw[RB][1];
-            load_rows<RB, 1, 1>(y, c * 2, sym * 2, pos, j0, n, raw);
+            load_rows<RB, 1>(y, c * 2, sym * 2, pos, j0, n, raw);
 #pragma unroll
             for (int jj = 0; jj < RB; ++jj) {
               const int j = j0 + jj;

@@ -360,6 +360,28 @@ def test_combine_every_top_k(dev, k, D, dtype):
     assert ((got_ds.double() - ds).abs() <= (D / 8 + 8) * 2 ** -23 * D ** 0.5 * 16).all()
 
 
+# Widths whose last step holds a whole first piece only, or cuts a lane's first or second piece;
+# rows further apart than they are wide (pieces stay aligned at odd widths)
+@pytest.mark.parametrize("D,pad,dtype", [(640, 0, torch.float16), (1004, 4, torch.bfloat16), (501, 11, torch.float16),
+                                         (300, 0, torch.float32), (387, 1, torch.float32), (1300, 0, torch.float16)])
+@pytest.mark.parametrize("k", [2, 7])
+def test_combine_partial_steps(dev, D, pad, dtype, k):
+    T, E = 37, 16
+    g = torch.Generator(device=dev).manual_seed(k * D)
+    idx = torch.rand(T, E, generator=g, device=dev).argsort(dim=1)[:, :k].contiguous()
+    _, inv, _, _, _ = moe.moe_route(idx, E)
+    y = torch.randn(T * k, D + pad, generator=g, device=dev).to(dtype)[:, :D]
+    sc = torch.rand(T, k, generator=g, device=dev)
+    pos, slot = inv.view(T, k).long().sort(dim=1)
+    out, total = torch.zeros(T, D, device=dev), torch.zeros(T, D, device=dev)
+    for j in range(k):
+        rows = y[pos[:, j]].float()
+        out = out + rows * sc.gather(1, slot[:, j:j + 1])
+        total = total + rows
+    assert torch.equal(moe.moe_combine(y, sc, inv), out)
+    assert torch.equal(moe.moe_gather_sum(y, inv, k, torch.float32), total)
+
+
 def test_traced_dispatch_computes_on_other_inputs(dev):
     """torch.jit.trace records the operators, so the traced chain runs them on whatever it is
     given (not the memory their outputs happened to have)."""
