@@ -1871,14 +1871,19 @@ bool big_offsets_fit(int64_t lda, int64_t ldb, int64_t klen, int64_t ssam, int64
   return 255 * lda + klen < lim && 255 * ldb + klen < lim && (255 * ssam + (nkb - 1) * ssak + 1) * 4 < lim;
 }
 
-// Whether a grid of 256 x 256 tiles leaves so many CUs idle in its last round that the 128 x
-// 128 and smaller tiles finish first: up to half a round (whose 128 x 128 tiles, two a CU, are
-// one round), or an eighth past a full one.  us, 256 x 256 / smaller tiles, by tiles on 256 CUs:
+// Whether a grid of 256 x 256 tiles of nk K blocks leaves so many CUs idle in its last round that
+// the 128 x 128 and smaller tiles finish first: up to half a round (whose 128 x 128 tiles, two a CU,
+// are one round), or an eighth past a full one.  us, 256 x 256 / smaller tiles, by tiles on 256 CUs:
 // 64 (4096, 1024, 1024) 14.9 / 11.5 and (2048, 2048, 2048) 24.5 / 16.0; 128 (4096, 2048, 4096) 44.5 /
 // 40.9; 136 (4352, 2048, 4096) 44.4 / 57.5; 160 (2560, 4096, 1024) 17.2 / 22.6; 264 (8448, 2048, 4096)
 // 96.6 / 90.2; 288 (9216, 2048, 4096) 96.0 / 93.3; 320 (10240, 2048, 4096) 94.6 / 99.2.
-bool rounds_sparse(int64_t tiles, int64_t ncu) {
-  return tiles * 2 <= ncu || (tiles > ncu && tiles * 8 <= ncu * 9);
+// With few K blocks C is most of a tile and the larger one stores it faster: 120 (3072, 2560, K)
+// with K = 128, 512, 768, 1024: 8.2 / 9.0, 11.1 / 11.9, 13.4 / 13.9, 16.1 / 16.2; 64 (4096, 1024, K) with 128,
+// 256: 7.3 / 7.8, 8.6 / 7.8; 32 (2048, 1024, 128): 6.7 / 5.1; 264 (8448, 2048, K) with 128, 256: 17.0 / 17.8,
+// 19.8 / 19.4.
+bool rounds_sparse(int64_t tiles, int64_t ncu, int64_t nk) {
+  if (tiles > ncu) return tiles * 8 <= ncu * 9 && nk >= 2;
+  return tiles * 8 <= ncu || (tiles * 4 <= ncu && nk >= 2) || (tiles * 2 <= ncu && nk >= 8);
 }
 
 }  // namespace
@@ -1921,7 +1926,7 @@ int cin_gemm_fp8_bs(const uint8_t* A, int64_t lda, const float* sa, int64_t ssam
   const uint32_t ncu = (uint32_t)cin_device_cus();
   const bool tile_fits = gt::offsets_fit(128, lda, ldb, K, ssam, ssak);
   if (K % big::TK == 0 && M >= big::TM && N >= big::TN && N % 128 == 0 && big_offsets_fit(lda, ldb, K, ssam, ssak) &&
-      !(tile_fits && rounds_sparse(cdiv(M, big::TM) * cdiv(N, big::TN), ncu))) {
+      !(tile_fits && rounds_sparse(cdiv(M, big::TM) * cdiv(N, big::TN), ncu, K / 128))) {
     const uint32_t tm = (uint32_t)cdiv(M, big::TM), tn = (uint32_t)cdiv(N, big::TN);
     if (tm * tn > ncu) {
       // more tiles than CUs: the persistent walk, whose next tile's DMA overlaps this tile's
@@ -1997,7 +2002,7 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
     CIN_CHECK_ARG(big_ok || (cdiv(T, 128) + E) * cdiv(N, 128) < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
     if (E == 1) {
       // one expert: as the dense product of the same shape
-      if (!big_ok || rounds_sparse(cdiv(T, big::TM) * cdiv(N, big::TN), ncu)) {
+      if (!big_ok || rounds_sparse(cdiv(T, big::TM) * cdiv(N, big::TN), ncu, K / 128)) {
         with_tile(T, N, ncu, launch);
         return cin_check_launch("grouped_gemm_fp8");
       }
@@ -2090,7 +2095,7 @@ int cin_grouped_gemm_fp8_wgrad(const uint8_t* A, int64_t lda, const float* sa, i
   const int64_t tiles = E * tm * tn;
   const bool tiles_fit = gt::offsets_fit(128, lda, ldb, tcap, ssam, ssak);
   const int by_load = tiles_fit && tiles <= 4 * cus && T >= 256 * E;
-  if (tiles_fit && (E == 1 ? rounds_sparse(tiles, cus) : 2 * tiles <= cus)) {
+  if (tiles_fit && (E == 1 ? rounds_sparse(tiles, cus, cdiv(T, 128)) : 2 * tiles <= cus)) {
     const auto launch = [&](auto cfg) {
       using C_ = decltype(cfg);
       const uint32_t tm_ = (uint32_t)cdiv(N, C_::TM), tn_ = (uint32_t)cdiv(K, C_::TN);
