@@ -666,30 +666,8 @@ __device__ __forceinline__ void tile_body(const Tile& T, int64_t lda, int64_t ss
   store_tile(T, acc, smu, wave, lane, c_dtype, ldc);
 }
 
-// XCD-aware order: workgroup b runs on XCD b % 8; give each XCD a contiguous run of
-// tile ids (n fastest) so its CUs share A row panels and B in their L2.
-// Tile index v -> (tm, tn): groups of GM m-tiles swept n by n, m fastest, so the 32 tiles
-// an XCD runs at once share GM A row panels and 32 / GM B column panels.  Measured
-// alternating in one process: GM = 8 took the config-3 grouped gate/up GEMM 4055 -> 3991
-// us and its dgrad 4486 -> 4370 us against GM = 4 (down the same; GM = 16 was 1.5-2%
-// slower than 8 on all three); the grouped wgrad and
-// the config-4 dgrad keep GM = 4 (8 was 0.6% slower, and the same).  In the one-round
-// kernel, GM = 4 took the config-4 wgrad (8 x 28 tiles) 125.5 -> 113.1 us against whole
-// m rows per XCD, where every XCD read all of B; config 2 maps the same either way.
-template <uint32_t GM>
-__device__ inline void raster(uint32_t v, uint32_t tiles_m, uint32_t tiles_n, uint32_t& tm, uint32_t& tn) {
-  const uint32_t gsz = GM * tiles_n;
-  const uint32_t grp = v / gsz, first = grp * GM;
-  const uint32_t gm = tiles_m - first < GM ? tiles_m - first : GM;
-  const uint32_t w = v - grp * gsz;
-  tm = first + w % gm;
-  tn = w / gm;
-}
-
-__device__ inline uint32_t xcd_remap(uint32_t b, uint32_t G) {
-  const uint32_t Gfull = G & ~7u;
-  return b < Gfull ? (b & 7u) * (Gfull >> 3) + (b >> 3) : b;
-}
+using cin::raster;
+using cin::xcd_remap;
 
 // Every tile is a full block inside the operands (M, N >= 256, N % 128 == 0): the
 // last tile of a row/column shifts back onto its neighbour and stores only the
@@ -1730,12 +1708,11 @@ __global__ __launch_bounds__(C::kThreads) void k_grouped_gemm_fp8_tile(
     int64_t ssak, const uint8_t* __restrict__ B, int64_t sbe, int64_t ldb,
     const float* __restrict__ sb, int64_t ssbe, int64_t ssbn, int64_t ssbk,
     const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t Tn,
-    int64_t N, int K, void* Cp, int c_dtype, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n, uint32_t walk) {
+    int64_t N, int K, void* Cp, int c_dtype, int64_t ldc, uint32_t tiles_n, uint32_t walk) {
   __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
-  uint32_t tm, tn;
-  big::raster<4>(big::xcd_remap(blockIdx.x, gridDim.x), tiles_m, tiles_n, tm, tn);
+  uint32_t tn;
   int64_t e, row0, row_end;
-  if (!find_row_tile<C::TM>(starts, ends, E, Tn, tm, e, row0, row_end)) return;  // the whole workgroup
+  if (!find_tile<C::TM>(starts, ends, E, Tn, tiles_n, e, row0, row_end, tn)) return;  // the whole workgroup
   const int64_t n0 = (int64_t)tn * C::TN;
   gt::Tile t;
   t.A = A + row0 * lda;
@@ -1997,7 +1974,7 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
       const int64_t tm = cdiv(T, C_::TM) + E - 1, tn = cdiv(N, C_::TN);
       const auto k = K % 128 == 0 ? k_grouped_gemm_fp8_tile<C_, false> : k_grouped_gemm_fp8_tile<C_, true>;
       hipLaunchKernelGGL(k, (unsigned)(tm * tn), C_::kThreads, 0, s, A, lda, sa, ssam, ssak, B, sbe, ldb, sb, ssbe, ssbn,
-                         ssbk, starts, ends, E, T, N, (int)K, C, c_dtype, ldc, (uint32_t)tm, (uint32_t)tn, walk);
+                         ssbk, starts, ends, E, T, N, (int)K, C, c_dtype, ldc, (uint32_t)tn, walk);
     };
     CIN_CHECK_ARG(big_ok || (cdiv(T, 128) + E) * cdiv(N, 128) < ((int64_t)1 << 31), "grouped_gemm_fp8: grid too large");
     if (E == 1) {

@@ -157,18 +157,12 @@ template <class C, int ADT, int BDT, bool ALIGNED>
 __global__ __launch_bounds__(C::kThreads, 2) void k_grouped_gemm_f16_tile(
     const void* __restrict__ A, int64_t lda, const void* __restrict__ B, int64_t sbe, int64_t ldb,
     const int64_t* __restrict__ starts, const int64_t* __restrict__ ends, int64_t E, int64_t T,
-    int64_t N, int64_t K, _Float16* __restrict__ Cp, int64_t ldc, uint32_t tiles_m, uint32_t tiles_n) {
+    int64_t N, int64_t K, _Float16* __restrict__ Cp, int64_t ldc, uint32_t tiles_n) {
   __shared__ __attribute__((aligned(128))) uint8_t smem[C::kBytes];
   constexpr int MT = C::MT, NT = C::NT;
-  // workgroup b runs on XCD b % 8: each XCD takes a contiguous run of tiles, four row tiles
-  // (mostly one expert's) against one column tile after another
-  const uint32_t G = gridDim.x, Gf = G & ~7u, b0 = blockIdx.x;
-  const uint32_t b = b0 < Gf ? (b0 & 7u) * (Gf >> 3) + (b0 >> 3) : b0;
-  const uint32_t grp = b / (4 * tiles_n), first = grp * 4;
-  const uint32_t gm = tiles_m - first < 4 ? tiles_m - first : 4, w = b - grp * 4 * tiles_n;
-  const uint32_t tm = first + w % gm, tn = w / gm;
+  uint32_t tn;
   int64_t e, r0, r1;
-  if (!find_row_tile<C::TM>(starts, ends, E, T, tm, e, r0, r1)) return;  // the whole workgroup
+  if (!find_tile<C::TM>(starts, ends, E, T, tiles_n, e, r0, r1, tn)) return;  // the whole workgroup
   const int nr = __builtin_amdgcn_readfirstlane((int)(r1 - r0 < C::TM ? r1 - r0 : C::TM));
   const int64_t n0 = (int64_t)tn * C::TN;
   const int nc = (int)(N - n0 < C::TN ? N - n0 : C::TN);
@@ -272,8 +266,7 @@ template <class C, int ADT, int BDT, bool ALIGNED>
 void launch_tile(const Args& a, hipStream_t s) {
   const int64_t tm = cdiv(a.T, C::TM) + a.E - 1, tn = cdiv(a.N, C::TN);
   hipLaunchKernelGGL((k_grouped_gemm_f16_tile<C, ADT, BDT, ALIGNED>), (unsigned)(tm * tn), C::kThreads, 0, s, a.A,
-                     a.lda, a.B, a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C, a.ldc, (uint32_t)tm,
-                     (uint32_t)tn);
+                     a.lda, a.B, a.sbe, a.ldb, a.starts, a.ends, a.E, a.T, a.N, a.K, a.C, a.ldc, (uint32_t)tn);
 }
 
 template <int ADT, int BDT>

@@ -297,6 +297,8 @@ def test_grouped_gemm_leaves_rows_outside_ranges(kern, dev, out_dtype):
     ([65, 31, 0, 63, 1, 97], 384, 1024),                 # 64 rows
     ([200, 0, 129, 90, 1], 100, 400),
     ([300, 700, 0, 128], 328, 144),                      # 128 rows
+    ([0] * 30 + [1] + [0] * 20 + [2], 384, 272),         # fewer tiles than XCDs, most workgroups surplus
+    ([1] + [0] * 90 + [7], 1000, 144),
 ])
 def test_grouped_tile_edges(kern, dev, counts, N, K):
     from cinnamon_amd import layers
