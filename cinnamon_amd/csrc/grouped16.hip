@@ -6,7 +6,8 @@
 // Operands are rounded to fp16 (round-to-nearest-even) as the reference's
 // a.to(tl.float16) / b.to(tl.float16) do, the products are summed in fp32 by
 // v_mfma_f32_16x16x32_f16, and the result is stored as fp16 (RNE).  One launch covers all
-// experts: a workgroup finds its (expert, row tile) from the device-side ranges, so there is no host synchronisation and no grid sized by the largest expert.
+// experts: a workgroup finds its (expert, row tile) from the device-side ranges, so there is
+// no host synchronisation and no grid sized by the largest expert.
 // Rows outside every expert range are not written (the reference returns torch.empty).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -281,7 +282,7 @@ void launch(const Args& a, hipStream_t s) {
     // 1024 (four rounds of 256 x 256): 217, 174 / 236, 208 / 297, 240; 16384 (two): 120, 109 / 120,
     // 105 / 151, 123; 8192 (one): 76, 67 / 69, 60 / 86, 69; 1024 (64 rows an expert): 37, 34 / 31, 24 /
     // 33, 19; 64: 37, 34 / 22, 17 / 22, 15.
-    if (a.T / 256 * cdiv(a.N, 256) >= 512)
+    if (a.T / 256 * cdiv(a.N, 256) >= 2 * (int64_t)cin_device_cus())
       launch_tile<W256, ADT, BDT, true>(a, s);
     else if (few)
       launch_tile<W64x128, ADT, BDT, true>(a, s);
