@@ -56,10 +56,14 @@ def _run_fp32_and_bf16(kern, dev, xq, xs, wq, ws):
     (1, 128, 128),
     (16368, 1024, 1024),  # config 5 MTP rows
     (4100, 4224, 512),    # more 256 x 256 tiles than CUs (persistent walk), last row and column shifted
-    (2304, 7296, 4096),   # persistent walk with the XCD-rotated K order (32 K blocks)
-    (8192, 2176, 384),    # 288 tiles (persistent walk), N % 256 = 128: the last column tile shifted back
+    (2304, 7296, 4096),   # 261 tiles of 256 x 256, an eighth past a round: 128 x 128 tiles
+    (8192, 2176, 384),    # 288 tiles, the same
     (6400, 5376, 256),    # 525 tiles: XCD-major ranges of 65 and 66 tiles, three rounds
-    (2560, 6912, 256),    # 270 tiles: ranges of 33 and 34 tiles, the last partly empty
+    (2560, 6912, 256),    # 270 tiles, 128 x 128 ones again
+    (4352, 4608, 2048),   # 306 tiles: persistent walk with the XCD-rotated K order (16 K blocks)
+    (8448, 2432, 384),    # 330 tiles (persistent walk), N % 256 = 128: the last column tile shifted back
+    (3328, 5888, 256),    # 299 tiles: ranges of 37 and 38 tiles, the last partly empty
+    (2300, 2176, 512),    # 81 tiles, too many for smaller ones at 4 K blocks: one round, both edges shifted
 ])
 def test_gemm_parity(kern, dev, M, N, K):
     xq, xs, wq, ws = _operands(M, N, K, seed=M + N + K)
@@ -81,7 +85,8 @@ def test_gemm_parity(kern, dev, M, N, K):
     (1000, 1000, 1168), (769, 1025, 528),                          # 64 x 64
     (1025, 1600, 1168), (2048, 1024, 512),                         # 64 x 64, two per CU
     (2047, 2040, 656), (4096, 1024, 1024),                         # 128 x 128
-    (2200, 2100, 272), (2049, 8191, 144), (4224, 2176, 384),       # 128 x 128, two per CU
+    (2200, 2100, 272), (2049, 8191, 144), (4096, 1920, 1024),      # 128 x 128, two per CU
+    (4224, 2176, 384),                             # (153 tiles of 256 x 256: one round of those)
 ])
 def test_gemm_tile_edges(kern, dev, M, N, K):
     xq, xs, wq, ws = _operands(M, N, K, seed=M + N + K)
@@ -311,6 +316,19 @@ def test_grouped_tile_edges(kern, dev, counts, N, K):
     assert torch.equal(y16.cpu(), y32.cpu().to(torch.bfloat16)), "bf16 output is not RNE(fp32 output)"
 
 
+@pytest.mark.parametrize("K", [272, 384])
+def test_grouped_rows_past_32_bit_offsets(kern, dev, K):
+    """Rows 16 MiB apart: past the lane offsets of the tiles, the 64-bit grouped kernel."""
+    from cinnamon_amd import layers
+    counts, N = [30, 0, 69, 1], 328
+    xq, xs, wq, ws, starts, ends = _grouped_case(counts, 384, K, seed=K)
+    far = torch.empty(sum(counts), (1 << 24) + 256, dtype=torch.uint8, device=dev)[:, :K]
+    far.copy_(xq.view(torch.uint8))
+    y = layers.fp8_grouped_gemm(far.view(torch.float8_e4m3fn), xs.to(dev), wq[:, :N].to(dev), ws.to(dev), starts.to(dev),
+                                ends.to(dev), out_dtype=torch.float32)
+    _check(y, orc.grouped_gemm_ref(xq, xs, wq[:, :N], ws, starts, ends), "grouped with distant rows")
+
+
 def _walk_order_ref(codes, sa, w, sb, counts, N, grid):
     """The grouped product bit for bit, its K blocks added in the order of the persistent walk:
     walk index v of the 256 x 256 tiles (groups of 8 row tiles, column by column) belongs to
@@ -411,12 +429,14 @@ def test_gemm_rows_past_32bit_tile_offsets(kern, dev):
 
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("pad", [1, 2, 4])
-def test_persistent_gemm_into_strided_c(kern, dev, out_dtype, pad):
-    """More tiles than CUs (9 x 29): the persistent walk, whose epilogue depends on C's
+@pytest.mark.parametrize("M,N", [(4352, 4608), (2560, 4096), (2304, 7296)])
+def test_persistent_gemm_into_strided_c(kern, dev, out_dtype, pad, M, N):
+    """17 x 18 tiles, more than CUs: the persistent walk, whose epilogue depends on C's
     alignment (fixed-count 16-bit or fp32 stores, or direct stores for rows that are not
-    aligned).  A C with row stride N + pad gets the same values as a contiguous C, bit for
-    bit (same kernel, same K order), and the padding columns are left alone."""
-    M, N, K = 2304, 7296, 512
+    aligned); 10 x 16: the one-round kernel; 9 x 29, just past a round: 128 x 128 tiles.  A C
+    with row stride N + pad gets the same values as a contiguous C, bit for bit (same kernel,
+    same K order), and the padding columns are left alone."""
+    K = 512
     g = torch.Generator(device=dev).manual_seed(21)
     xq, xs = kern.quantize_fp8_rowwise(torch.randn(M, K, device=dev, generator=g).to(torch.bfloat16))
     wq, ws = kern.quantize_fp8_blockwise((torch.randn(N, K, device=dev, generator=g) * 0.02).to(torch.bfloat16))
@@ -456,13 +476,14 @@ def _special_scale_patterns():
     return p
 
 
-@pytest.mark.parametrize("M,N", [(512, 512), (4352, 4096)])
+@pytest.mark.parametrize("M,N", [(512, 512), (2560, 4096), (4352, 4096)])
 @pytest.mark.parametrize("path", ["dense_bf16", "grouped_bf16", "grouped_f16"])
 def test_gemm_half_output_rounding_special_values(kern, dev, M, N, path):
     """The 16-bit epilogues round the fp32 result exactly as the fp32 output rounded to
-    nearest even.  Dense: the one-round LDS-staged tile at 2 x 2 tiles, the persistent
-    16-byte stores and its last-tile LDS path at 17 x 16 tiles; grouped (one expert over
-    every row): the persistent walk at both sizes, bf16 and fp16.  One K block in which row
+    nearest even.  Dense: the small tiles' stores at 2 x 2 tiles, the one-round LDS-staged tile
+    at 10 x 16, the persistent 16-byte stores and its last-tile LDS path at 17 x 16 (past a round,
+    but with a single K block); grouped (one expert over every row): the small tiles, then the
+    persistent walk at both larger sizes, bf16 and fp16.  One K block in which row
     m of A and row n of B hold a single non-zero code, so C[m, n] = b_n * sa[m] with b_n
     mostly a power of two, which carries the chosen scale bit patterns (ties, denormals,
     overflow, NaN payloads) into C unchanged.  bf16: bit-exact against the integer RNE of

@@ -340,10 +340,7 @@ def _many_expert_counts(E, T, seed):
 
 @pytest.mark.parametrize("E,T", [(256, 20000), (600, 20000), (4096, 30000), (4100, 3000)])
 def test_grouped_forward_many_experts(kern, dev, E, T):
-    """256 experts (DeepSeek-V3's count): the persistent kernel's prefix-table lookup, several
-    tiles per workgroup; 600 and 4096 experts: each of the 512 threads that build the prefix
-    table sums the tile counts of 2 and 8 experts; 4100 experts: beyond the LDS prefix table,
-    the one-tile-per-workgroup kernel."""
+    """Few rows an expert: the short tiles, whose waves look the experts up 64 at a time."""
     from cinnamon_amd import layers
     counts = _many_expert_counts(E, T, seed=E)
     starts, ends = _ranges(counts)
@@ -421,10 +418,9 @@ def test_grouped_wgrad_both_kernels(kern, dev, E):
 
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_grouped_wgrad_direct_epilogue(kern, dev, out_dtype):
-    """An expert stride (sce) that is not a multiple of 4 elements sends the persistent wgrad
-    to its direct-store epilogue: every expert's dW equals the contiguous call's bit for bit
-    (same kernel walk, same K order), and the element between two experts' blocks is left
-    alone."""
+    """An expert stride (sce) that is not a multiple of 4 elements: every expert's dW equals the
+    contiguous call's bit for bit (same tiles, same K order), and the element between two
+    experts' blocks is left alone.  (16 tiles of 256 x 256: the 128 x 128 ones take it.)"""
     from cinnamon_amd import _lib, layers
     E, T, N, K = 8, 3000, 256, 384
     counts = [700, 0, 128, 1, 555, 64, 900, 652]
@@ -449,8 +445,9 @@ def test_grouped_wgrad_direct_epilogue(kern, dev, out_dtype):
         assert float(buf[e * sce + N * K]) == 5.0, f"the element after expert {e}'s block was written"
 
 
-# The 128 x 128 wgrad tiles: partial tiles, experts in size order (up to 64) and in expert order
-@pytest.mark.parametrize("E,T,N,K", [(64, 5000, 304, 256), (70, 5000, 304, 384), (3, 700, 256, 640)])
+# The 128 x 128 wgrad tiles: partial tiles, experts in size order (up to 64) and in expert order;
+# and (280 tiles of 256 x 256) the persistent walk with more than 64 experts
+@pytest.mark.parametrize("E,T,N,K", [(64, 5000, 304, 256), (100, 5000, 256, 256), (3, 700, 256, 640), (70, 5000, 304, 384)])
 def test_grouped_wgrad_tiles(kern, dev, E, T, N, K):
     from cinnamon_amd import layers
     counts = _many_expert_counts(E, T, seed=E)
@@ -474,7 +471,8 @@ def test_grouped_wgrad_tiles(kern, dev, E, T, N, K):
 
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
 def test_grouped_wgrad_persistent_direct_epilogue(kern, dev, out_dtype):
-    """The same with more than four rounds of 256 x 256 tiles, which the persistent walk takes."""
+    """The same with more than four rounds of 256 x 256 tiles: the persistent walk, which that
+    stride sends to its direct-store epilogue, against the dense product of each expert's operands."""
     from cinnamon_amd import _lib, layers
     E, T, N, K = 8, 1500, 3072, 2944
     starts, ends = _ranges([700, 0, 128, 1, 300, 64, 7, 300])
@@ -496,14 +494,24 @@ def test_grouped_wgrad_persistent_direct_epilogue(kern, dev, out_dtype):
     for e in range(E):
         assert torch.equal(buf[e * sce:e * sce + N * K].view(N, K), want[e]), f"expert {e}"
         assert float(buf[e * sce + N * K]) == 5.0, f"the element after expert {e}'s block was written"
-    # expert 0's block (700 tokens, 768 padded) against the dense product of its operands
-    dense = kern.fp8_gemm_bs(qt[:, :768], st[:, :6], xbt[:, :768], xblk[:6].t(), torch.float32)
-    _check(want[0], dense.to(out_dtype).cpu(), "expert 0")
+    p = 0  # the expert's first padded token
+    for e, c in enumerate([700, 0, 128, 1, 300, 64, 7, 300]):
+        n = -(-c // 128) * 128
+        if n == 0:
+            assert torch.count_nonzero(want[e]) == 0, f"expert {e}"
+            continue
+        t, blk = slice(p, p + n), slice(p // 128, (p + n) // 128)
+        dense = kern.fp8_gemm_bs(qt[:, t], st[:, blk], xbt[:, t], xblk[blk].t(), torch.float32)
+        _check(want[e], dense.to(out_dtype).cpu(), f"expert {e}")
+        p += n
 
 
 @pytest.mark.parametrize("E,T", [(256, 40000), (600, 80000), (4096, 263000), (4100, 263000)])
 def test_grouped_forward_many_experts_long(kern, dev, E, T):
-    """The same with enough rows an expert for the 256-row tiles."""
+    """The same with enough rows an expert for the 256-row tiles.  256 experts (DeepSeek-V3's
+    count): the persistent kernel's prefix-table lookup, several tiles per workgroup; 600 and 4096
+    experts: each of the 512 threads that build the prefix table sums the tile counts of 2 and 8
+    experts; 4100 experts: beyond the LDS prefix table, the one-tile-per-workgroup kernel."""
     test_grouped_forward_many_experts(kern, dev, E, T)
 
 

@@ -109,11 +109,11 @@ def test_backward_triple_col_scales(dev, M, N, K):
         _same(ta, tb, what)
 
 
-@pytest.mark.parametrize("M,N,K", [(512, 768, 1024), (8192, 2176, 384)])
+@pytest.mark.parametrize("M,N,K", [(512, 768, 1024), (8192, 2176, 384), (2560, 4096, 384), (8448, 2432, 384)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
 def test_gemm_col_a_scales(dev, M, N, K, out_dtype):
-    """One-round (2 x 3 tiles) and persistent (32 x 9 tiles) GEMMs: column-major A scales
-    give the same output, bit for bit."""
+    """Small tiles (first two), one-round (10 x 16 tiles) and persistent (33 x 10 tiles) GEMMs:
+    column-major A scales give the same output, bit for bit."""
     x = _x(M, K, torch.bfloat16, dev, seed=7)
     w = _x(N, K, torch.bfloat16, dev, seed=8) * 0.02
     xq, s_row = kernels.quantize_fp8_rowwise(x)
