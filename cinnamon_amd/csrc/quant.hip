@@ -542,7 +542,8 @@ __device__ inline void t8x8(const uint32_t (&rows)[8][2], uint32_t (&cols)[8][2]
 // one is quantized; the two sets alternate, so no register copy waits on a load.
 //
 // Column blocks that run past the last column (N % 128 != 0) go to a second launch with
-// EDGE = true, whose element-wise loads and stores are masked.  The main launch addresses
+// EDGE = true: whole 8-column pieces move as vectors there too, the one that the edge cuts
+// element by element.  The main launch addresses
 // a tile through buffer descriptors whose range ends after the tile's last valid row:
 // rows past it read as zero and are not written, with no per-row test.
 // ---------------------------------------------------------------------------
@@ -888,7 +889,7 @@ __device__ __forceinline__ float row_scales8(const float (&ra)[8], float floor_v
 }
 
 // Row-major code output of a tile: main launch through a buffer descriptor (rows past
-// the tile are out of range), EDGE through masked byte stores.
+// the tile are out of range), EDGE as 8-byte stores, byte by byte where the edge cuts.
 template <bool EDGE>
 struct RowOut {
   __amdgpu_buffer_rsrc_t r;
@@ -2570,6 +2571,7 @@ int cin_transpose_u8(const uint8_t* src, int64_t R, int64_t C, int64_t lds, uint
   CIN_CHECK_ARG(R >= 0 && C >= 0, "transpose_u8: negative shape");
   if (R == 0 || C == 0) return CIN_OK;
   CIN_CHECK_ARG(src && dst && lds >= C && ldd >= R, "transpose_u8: bad pointer or stride");
+  // (the entry's limit, half of what the grid of 128-row tiles could take)
   CIN_CHECK_ARG(cdiv(R, 64) < 65536, "transpose_u8: too many rows");
   hipStream_t s = static_cast<hipStream_t>(stream);
   dim3 grid((unsigned)cdiv(C, 128), (unsigned)cdiv(R, 128));

@@ -14,7 +14,7 @@ Replaced reference items (src/kernels.py):
   dequantize_fp8_rowwise    :262-281  -> cin_dequant (fp32 out)
   dequantize_fp8            :284-314  -> cin_dequant (bf16 out)
   fp8_matmul_dsv3           :667-702  -> cin_gemm_fp8_bs
-  FP8MatmulFunction         :731-794  -> cin_quant_fwd + cin_quant_dual + cin_requant_row_to_block + GEMMs
+  FP8MatmulFunction         :731-794  -> cin_quant_fwd + cin_quant_backward_padded + GEMMs
   FP8Linear                 :797-840
   convert_to_fp8            :843-905
   moe_grouped_gemm          :526-581  -> cin_grouped_gemm_f16 (unquantized, fp16 MFMA)
@@ -666,7 +666,8 @@ class FP8MatmulFunction(torch.autograd.Function):
     Forward quantizes x row-wise and the weight block-wise (emitting the transposed
     weight codes for dgrad) and runs one GEMM.  Backward quantizes dY once into row
     tiles and dY^T row tiles and re-quantizes the saved x codes into transposed 128x128
-    blocks, all in one launch (cin_quant_backward), and runs the dgrad and wgrad GEMMs,
+    blocks, padded with zeros to whole 128-token blocks, all in one launch
+    (cin_quant_backward_padded), and runs the dgrad and wgrad GEMMs,
     with the same operands and rounding steps as the reference.
     """
 
