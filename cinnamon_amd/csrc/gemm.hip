@@ -1989,8 +1989,8 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
     } else {
       // Few rows an expert: the product streams every expert's codes for a fraction of a 256-
       // row tile, so short tiles, three workgroups a CU.  us, 32 x 128 / 64 x 128 / 128 x 128 / 256 x
-      // 256 tiles at T, E, N, K: 512, 32, 4096, 7168: 224 / 239 / 254 / 274; 1024: 262 / 249 / 281 /
-      // 275; 2048: 352 / 289 / 275 / 274.  With up to 128 rows an expert the 256 x 256 tiles are
+      // 256 tiles at T, E, N, K: 512, 32, 4096, 7168: 224 / 239 / 254 / 274 (in a loop on the same
+      // operands 175-185 and, the last, 235); 1024: 262 / 249 / 281 / 275; 2048: 352 / 289 / 275 / 274.  With up to 128 rows an expert the 256 x 256 tiles are
       // half empty; they still win where they fill the chip (4096, 32, 4096, 7168: 418 against
       // 347), not where about T / 256 + E / 2 row tiles do not (2048, 16, 2048, 1024: 19.8 against
       // 27.5; 8192, 64, 1024, 512: 28.9 against 35.8).
