@@ -128,3 +128,15 @@ def test_opcheck_operators(dev):
     for save in (True, False):
         torch.library.opcheck(ops.indexer_scores_fp8_q.default, (qi, args[2], ksi, wi, 0.125, save),
                               test_utils=f8)
+
+
+@pytest.mark.parametrize("tokens", [300, 16384])
+def test_opcheck_padded_backward_quantization(dev, tokens):
+    """Shapes and strides of the shape function and of the launch, with and without the gap
+    between transposed rows that lie a multiple of 16 KiB apart."""
+    g = torch.Generator(device=dev).manual_seed(tokens)
+    xq, xs = kernels.quantize_fp8_rowwise(torch.randn(tokens, 256, device=dev, generator=g).to(torch.bfloat16))
+    gy = torch.randn(tokens, 128, device=dev, generator=g).to(torch.bfloat16)
+    op = torch.ops.cinnamon_amd.quant_bwd_padded.default
+    torch.library.opcheck(op, (gy, xq, xs, False), test_utils=("test_faketensor",))
+    assert op(gy, xq, xs, False)[2].stride(0) % 16384 != 0
