@@ -629,7 +629,12 @@ void with_k(int64_t k, F launch) {
 // Waves per token of the combine and the gather sum: one per step of 128 16-byte pieces (one
 // in all where the grid could not hold them).  16384 tokens, k 8, 7168 columns: 466 and 395 us,
 // with one wave a token 515 and 433.
-int token_waves(int64_t T, int64_t N, int dtype) {
+// Each wave sorts the token's positions anew: past k = 8, where that is much of a step's work, fp32
+// rows (half the columns a step) take one wave a token once those fill the chip: 4096 tokens, k 9,
+// 1024 / 2816 columns, gather sum 28.5 / 102 us, with a wave per step 32.5 / 108.  (16-bit rows lose at
+// most 1% with a wave per step.)
+int token_waves(int64_t T, int64_t k, int64_t N, int dtype) {
+  if (k > 8 && dtype == CIN_DT_F32 && T >= 4 * (int64_t)cin_device_cus()) return 1;
   const int64_t steps = cdiv(N, dtype == CIN_DT_F32 ? 512 : 1024);
   return steps < (1 << 30) && cdiv(T * steps * 64, kRT) < ((int64_t)1 << 31) ? (int)steps : 1;
 }
@@ -733,7 +738,7 @@ int cin_moe_gather_sum(const void* g, int g_dtype, int64_t sgm, const int32_t* i
   if (T == 0 || N == 0) return CIN_OK;
   CIN_CHECK_ARG(g && inv && out && sgm >= N && som >= N, "moe_gather_sum: bad pointers or strides");
   CIN_CHECK_ARG(cdiv(T * 64, kRT) < ((int64_t)1 << 31), "moe_gather_sum: grid too large");
-  const int nch = token_waves(T, N, g_dtype);
+  const int nch = token_waves(T, k, N, g_dtype);
   const unsigned grid = (unsigned)cdiv(T * nch * 64, kRT);
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define CIN_GS(GT, OT)                                                                                         \
@@ -769,7 +774,7 @@ int cin_moe_combine(const void* y, int y_dtype, int64_t sym, const void* scores,
   CIN_CHECK_ARG(y && scores && inv && out && sym >= N && som >= N && ssm >= k,
                 "moe_combine: bad pointers or strides");
   CIN_CHECK_ARG(cdiv(T * 64, kRT) < ((int64_t)1 << 31), "moe_combine: grid too large");
-  const int nch = token_waves(T, N, y_dtype);
+  const int nch = token_waves(T, k, N, y_dtype);
   const unsigned grid = (unsigned)cdiv(T * nch * 64, kRT);
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define CIN_COMB(YT, ST)                                                                                       \

@@ -364,9 +364,9 @@ def test_combine_every_top_k(dev, k, D, dtype):
 # rows further apart than they are wide (pieces stay aligned at odd widths)
 @pytest.mark.parametrize("D,pad,dtype", [(640, 0, torch.float16), (1004, 4, torch.bfloat16), (501, 11, torch.float16),
                                          (300, 0, torch.float32), (387, 1, torch.float32), (1300, 0, torch.float16)])
-@pytest.mark.parametrize("k", [2, 7])
-def test_combine_partial_steps(dev, D, pad, dtype, k):
-    T, E = 37, 16
+@pytest.mark.parametrize("k,T", [(2, 37), (7, 37), (9, 1100)])  # (past k = 8: one wave for all of a token's steps)
+def test_combine_partial_steps(dev, D, pad, dtype, k, T):
+    E = 16
     g = torch.Generator(device=dev).manual_seed(k * D)
     idx = torch.rand(T, E, generator=g, device=dev).argsort(dim=1)[:, :k].contiguous()
     _, inv, _, _, _ = moe.moe_route(idx, E)
