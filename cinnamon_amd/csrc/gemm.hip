@@ -1993,9 +1993,14 @@ int cin_grouped_gemm_fp8(const uint8_t* A, int64_t lda, const float* sa, int64_t
       // operands 175-185 and, the last, 235); 1024: 262 / 249 / 281 / 275; 2048: 352 / 289 / 275 / 274.  With up to 128 rows an expert the 256 x 256 tiles are
       // half empty; they still win where they fill the chip (4096, 32, 4096, 7168: 418 against
       // 347), not where about T / 256 + E / 2 row tiles do not (2048, 16, 2048, 1024: 19.8 against
-      // 27.5; 8192, 64, 1024, 512: 28.9 against 35.8).
+      // 27.5; 8192, 64, 1024, 512: 28.9 against 35.8).  Between half a round and a full one, with equal
+      // rows, they lose nothing up to K = 2048 and win past it (2016, 16, 4096, K = 2048, 4096, 7168: 34.4
+      // against 33.3, 78 against 61, 149 against 115; Zipf rows, which make more than a round of them, 46
+      // against 56, 87 against 107, 153 against 196).
       const int64_t rows = T / E;
-      const bool few = (rows < 64 || (rows <= 128 && (T / big::TM + E / 2) * cdiv(N, big::TN) <= ncu)) &&
+      const int64_t tn = cdiv(N, big::TN);
+      const bool idle = 2 * E * tn <= ncu || ((T / big::TM + E / 2) * tn <= ncu && K <= 2048);
+      const bool few = (rows < 64 || (rows <= 128 && idle)) &&
                        (cdiv(T, 32) + E) * cdiv(N, 128) < ((int64_t)1 << 31);
       if (few || !big_ok) {
         if (!few)

@@ -365,6 +365,7 @@ def _walk_order_ref(codes, sa, w, sb, counts, N, grid):
     ([3, 0, 33, 1, 64, 20, 0, 141], 512, 2176), ([20] * 14 + [1, 2], 384, 2048), ([70, 20, 1, 300], 640, 4224),
     ([5, 0, 280, 30] * 4 + [0] * 80, 768, 2048), ([9] * 40, 2048, 2048), ([40, 0, 30, 200], 512, 1920),
     ([300, 700, 0, 128], 640, 2176),
+    ([100] * 10, 3328, 2048), ([100] * 10, 3328, 2176), ([100] * 10, 1024, 2176),  # 65 to 128 rows: 64, 256, 64-row tiles
 ])
 def test_grouped_sums_do_not_depend_on_the_tile(kern, dev, counts, N, K):
     from cinnamon_amd import layers
